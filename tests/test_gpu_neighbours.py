@@ -148,6 +148,33 @@ def test_rmsnorm_matches_oracle(torch, okq, orc, rows, hidden):
     assert ok, info
 
 
+@pytest.mark.parametrize("rows,hidden,off", [(1, 4, 0), (3, 252, 0), (2, 4096, 0), (2, 4100, 0), (33, 4096, 0),
+                                             (1, 8192, 0), (2, 8196, 0), (2, 16384, 0), (1, 16388, 0), (2, 4098, 0),
+                                             (2, 4096, 1)])
+def test_rmsnorm_at_the_edges_of_its_kernels(torch, okq, rows, hidden, off):
+    """One, two and four float4s per thread, partly filled waves, and what the
+    loop kernel takes (longer rows, lengths and addresses off a float4).  The
+    sum of squares is a tree of fewer than 20 roundings up to 16384 values
+    (the loop kernel: 16388 / 256 + 8 = 73), the rest a handful: against
+    float64 within 80 * 2^-24 of the value, in place as well."""
+    print(f"[gpu] rmsnorm edges rows={rows} hidden={hidden} off={off}", flush=True)
+    rng = np.random.default_rng(rows + hidden)
+    x = rng.normal(0, 2, (rows, hidden)).astype(np.float32)
+    w = rng.normal(0, 1, hidden).astype(np.float32)
+    buf = torch.zeros(rows * hidden + off, device="cuda")
+    buf[off:] = _dev(torch, x.reshape(-1))
+    wd, out = _dev(torch, w), torch.full((rows * hidden + off,), float("nan"), device="cuda")
+    p = buf.data_ptr() + 4 * off
+    okq.call("okq_rmsnorm", p, rows, hidden, wd.data_ptr(), 1e-5, out.data_ptr() + 4 * off, _stream(torch))
+    okq.call("okq_rmsnorm", p, rows, hidden, wd.data_ptr(), 1e-5, p, _stream(torch))
+    torch.cuda.synchronize()
+    x64 = x.astype(np.float64)
+    want = x64 / np.sqrt((x64 * x64).mean(1, keepdims=True) + np.float64(np.float32(1e-5))) * w
+    got = out.cpu().numpy()[off:].reshape(rows, hidden)
+    assert (np.abs(got - want) <= 80 * 2.0 ** -24 * np.abs(want)).all()
+    assert (buf.cpu().numpy()[off:].view(np.uint32) == got.reshape(-1).view(np.uint32)).all()
+
+
 def test_rmsnorm_reference_kats_on_gpu(torch, okq):
     import json
     import os
