@@ -35,8 +35,10 @@ hipError_t launch_bf16_to_f32(const uint16_t *src, int64_t n, float *dst, hipStr
 
 // Row gather: out[j, :] = dequant(W row ids[j]) for j < n (ids in host memory,
 // each < the weight's row count).  Row ids ride in the kernel arguments,
-// kGatherMaxIds per launch.
-constexpr int kGatherMaxIds = 480;
+// kGatherMaxIds per launch: 3,840 bytes, so that with the other arguments a
+// launch stays below the 4 KB that kernel arguments may take, and a prompt of
+// up to 960 tokens is one launch.
+constexpr int kGatherMaxIds = 960;
 struct GatherIds {
   uint32_t id[kGatherMaxIds];
 };

@@ -86,6 +86,25 @@ def test_dequant_bit_exact_on_random_bytes(torch, okq, orc, t):
     assert (got[finite].view(np.uint32) == want[finite].view(np.uint32)).all()
 
 
+@pytest.mark.parametrize("t", O.GATHER_TYPES)
+@pytest.mark.parametrize("n", [256, 768, 3328, 4096, 4352, 12032])
+def test_dequant_bit_exact_around_the_workgroup_size(torch, okq, orc, t, n):
+    """A workgroup expands 4096 elements: fewer, exactly as many, one block
+    more and ragged tails, into a destination 4 bytes off a float4 and from a
+    source at the format's minimum alignment; nothing is written past n."""
+    print(f"[gpu] dequant n={n} type={t}", flush=True)
+    rng = np.random.default_rng(n + t)
+    blocks = rng.integers(0, 256, n // O.BLOCK_ELEMS[t] * O.BLOCK_BYTES[t], dtype=np.uint8)
+    off = 16 if t == O.Q4_K else 2
+    src = torch.zeros(blocks.size + off, dtype=torch.uint8, device="cuda")
+    src[off:] = _dev(torch, blocks)
+    out = torch.full((n + 5,), 7.0, dtype=torch.float32, device="cuda")
+    okq.call("okq_dequantize", t, src.data_ptr() + off, n, out.data_ptr() + 4, _stream(torch))
+    got = _host(out)
+    assert _same_bits(got[1:n + 1], orc.dequantize(t, blocks, n)).all()
+    assert got[0] == 7.0 and (got[n + 1:] == 7.0).all()
+
+
 @pytest.mark.parametrize("t", TYPES)
 def test_dequant_bit_exact_on_quantized_normal(torch, okq, orc, t):
     n = 4096 * 64
