@@ -33,7 +33,8 @@ EXTRA = {"okq_prep.hip": ["-ffp-contract=off"], "okq_gemv.hip": ["-ffp-contract=
          "okq_gemm_wide.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
          "okq_gemm_pair.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
          "okq_gemm_q8.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
-         "okq_gemm_q6.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+         "okq_gemm_q6.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+         "okq_gemm_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
 def sources():

@@ -96,10 +96,14 @@ __device__ __forceinline__ void prep_chunk(const float v[8], int s, bool ok, int
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const float w = ldexpf(v[i], -s);
-    t += w;
     const _Float16 h = (_Float16)w;
+    const _Float16 l = (_Float16)(w - (float)h);
     hv[i] = h;
-    lv[i] = (_Float16)(w - (float)h);
+    lv[i] = l;
+    // two planes: the sum is of what they hold, so that the min term meets the
+    // same rounded activations as the products (Q4_K, 512 x 4096 -> 14336:
+    // 4.9e-7 -> 4.7e-7 from float64)
+    t += kF32 ? (float)h + (float)l : w;
   }
   t += dpp_row_f<0xB1>(t);  // quad_perm 1,0,3,2
   t += dpp_row_f<0x4E>(t);  // quad_perm 2,3,0,1
@@ -158,12 +162,17 @@ __device__ __forceinline__ uint32_t abs_bits(float v) { return as_u32(v) & 0x7ff
 // x_k * W[o, k] over the row's non-finite positions k, then + bias[o]:
 // NaN where a product is NaN or infinities of both signs meet, the
 // infinity otherwise -- the reference's own values.
+// (of every matrix that the pre-pass serves)
 struct PrepIeee {
   const uint8_t *w;
   const float *bias;
   float *y;
   size_t row_bytes;
   int type, N;
+};
+struct PrepIeees {
+  PrepIeee mat[kPrefillMats];
+  int count;
 };
 constexpr int kIeeeCap = 1024;  // non-finite positions listed in LDS; more: every column scans the row
 
@@ -175,7 +184,7 @@ __device__ __forceinline__ float x_at(const void *X, int64_t i) {
 __device__ __forceinline__ bool non_finite(float v) { return !(fabsf(v) <= 3.4028235e38f); }
 
 template <bool kF32>
-__device__ void prep_ieee_row(const void *__restrict__ X, int m, int K, const PrepIeee &P, int tid) {
+__device__ void prep_ieee_row(const void *__restrict__ X, int m, int K, const PrepIeees &Ps, int tid) {
   __shared__ int cnt;
   __shared__ int pos[kIeeeCap];
   if (tid == 0) cnt = 0;
@@ -188,19 +197,22 @@ __device__ void prep_ieee_row(const void *__restrict__ X, int m, int K, const Pr
     }
   __syncthreads();
   const int n = cnt;
-  for (int o = tid; o < P.N; o += 256) {
-    const uint8_t *wrow = P.w + (size_t)o * P.row_bytes;
-    float acc = 0.0f;
-    if (n <= kIeeeCap) {
-      for (int j = 0; j < n; ++j)
-        acc = __fadd_rn(acc, __fmul_rn(x_at<kF32>(X, row + pos[j]), deq_elem(P.type, wrow, (uint32_t)pos[j])));
-    } else {
-      for (int k = 0; k < K; ++k) {
-        const float v = x_at<kF32>(X, row + k);
-        if (non_finite(v)) acc = __fadd_rn(acc, __fmul_rn(v, deq_elem(P.type, wrow, (uint32_t)k)));
+  for (int i = 0; i < Ps.count; ++i) {
+    const PrepIeee &P = Ps.mat[i];
+    for (int o = tid; o < P.N; o += 256) {
+      const uint8_t *wrow = P.w + (size_t)o * P.row_bytes;
+      float acc = 0.0f;
+      if (n <= kIeeeCap) {
+        for (int j = 0; j < n; ++j)
+          acc = __fadd_rn(acc, __fmul_rn(x_at<kF32>(X, row + pos[j]), deq_elem(P.type, wrow, (uint32_t)pos[j])));
+      } else {
+        for (int k = 0; k < K; ++k) {
+          const float v = x_at<kF32>(X, row + k);
+          if (non_finite(v)) acc = __fadd_rn(acc, __fmul_rn(v, deq_elem(P.type, wrow, (uint32_t)k)));
+        }
       }
+      P.y[(size_t)m * P.N + o] = __fadd_rn(acc, P.bias ? P.bias[o] : 0.0f);
     }
-    P.y[(size_t)m * P.N + o] = __fadd_rn(acc, P.bias ? P.bias[o] : 0.0f);
   }
 }
 
@@ -211,7 +223,7 @@ template <bool kF32, int CH>
 __global__ __launch_bounds__(256) void gemm_prep_kernel(const void *__restrict__ X, int M, int K,
                                                         _Float16 *__restrict__ xhi, _Float16 *__restrict__ xlo,
                                                         h2 *__restrict__ xsum, float *__restrict__ rscale,
-                                                        PrepIeee ieee) {
+                                                        PrepIeees ieee) {
   __shared__ uint32_t red[4];
   const int m = (int)blockIdx.x;
   const int tid = (int)threadIdx.x;
@@ -1709,8 +1721,10 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restr
         const uint32_t off = z0 + d < ksplit ? ((uint32_t)(z0 + d) * total + i) * 4u : end;
         v[d] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0));
       }
+      float t = -0.0f;  // each batch of slices summed on its own
 #pragma unroll
-      for (int d = 0; d < KB; ++d) acc += v[d];
+      for (int d = 0; d < KB; ++d) t += v[d];
+      acc += t;
     }
     Y[(size_t)i] = __builtin_fmaf(acc, rs_m, bn);  // rs_m a power of two: the product is exact
   }
@@ -1723,16 +1737,36 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restr
 // splitk_reduce_kernel.  Per output the same operations in the same order:
 // the slice-order sum from -0.0, then acc * rscale + bias as one FMA (the
 // power-of-two scale makes the product exact, so this is the rounding of
-// the separate multiply and add).  Grid: 1024-column blocks x RR-row blocks.
+// the separate multiply and add).  Grid: the matrices' 1024-column blocks
+// x RR-row blocks; matrices that were computed in one launch share one
+// reduction (each launch costs ~4.5 us here however small).
 constexpr int kReduceRows = 2;  // rows per thread of splitk_reduce4_kernel
-template <int KB, int RR>
-__global__ __launch_bounds__(256) void splitk_reduce4_kernel(const float *__restrict__ part, int ksplit, int M, int N,
-                                                             const float *__restrict__ rscale,
-                                                             const float *__restrict__ bias, float *__restrict__ Y) {
-  const int n = ((int)blockIdx.x * 256 + (int)threadIdx.x) * 4;
+struct ReduceMat {
+  const float *part, *bias;
+  float *y;
+  int n, ks, bx0;  // outputs, slices, first column block
+};
+struct ReduceMats {
+  ReduceMat mat[kPrefillMats];
+};
+template <int KB, int RR, bool kOne>
+__global__ __launch_bounds__(256) void splitk_reduce4_kernel(ReduceMats mats, int M, const float *__restrict__ rscale) {
+  const int bx = (int)blockIdx.x;
+  const int mi = kOne ? 0
+                      : (int)(bx >= sarg(mats.mat[1].bx0)) + (int)(bx >= sarg(mats.mat[2].bx0)) +
+                            (int)(bx >= sarg(mats.mat[3].bx0));
+  const ReduceMat &mt = mats.mat[mi];
+  auto arg = [](auto v) {  // fields at a computed index come in one batch of scalar loads
+    if constexpr (kOne) return v;
+    else return sarg(v);
+  };
+  const int N = arg(mt.n), ksplit = arg(mt.ks);
+  const float *const bias = arg(mt.bias);
+  float *const Y = arg(mt.y);
+  const int n = ((bx - (kOne ? 0 : arg(mt.bx0))) * 256 + (int)threadIdx.x) * 4;
   if (n >= N) return;
   const uint32_t total = (uint32_t)M * (uint32_t)N, end = (uint32_t)ksplit * total * 4u;
-  const Rsrc rs = make_rsrc(part, end);
+  const Rsrc rs = make_rsrc(arg(mt.part), end);
   const int m0 = (int)blockIdx.y * RR;
   f4 acc[RR];
 #pragma unroll
@@ -1748,17 +1782,20 @@ __global__ __launch_bounds__(256) void splitk_reduce4_kernel(const float *__rest
         v[r][d] = bload4(rs, in ? ((uint32_t)(z0 + d) * total + i) * 4u : end);
       }
 #pragma unroll
-    for (int r = 0; r < RR; ++r)
+    for (int r = 0; r < RR; ++r) {  // each batch of slices summed on its own
+      f4 t{-0.0f, -0.0f, -0.0f, -0.0f};
 #pragma unroll
       for (int d = 0; d < KB; ++d) {
-        acc[r].x += __uint_as_float(v[r][d].x);
-        acc[r].y += __uint_as_float(v[r][d].y);
-        acc[r].z += __uint_as_float(v[r][d].z);
-        acc[r].w += __uint_as_float(v[r][d].w);
+        t.x += __uint_as_float(v[r][d].x);
+        t.y += __uint_as_float(v[r][d].y);
+        t.z += __uint_as_float(v[r][d].z);
+        t.w += __uint_as_float(v[r][d].w);
       }
+      acc[r].x += t.x, acc[r].y += t.y, acc[r].z += t.z, acc[r].w += t.w;
+    }
   }
-  const float b0 = bias ? bias[n] : 0.0f, b1 = bias ? bias[n + 1] : 0.0f;
-  const float b2 = bias ? bias[n + 2] : 0.0f, b3 = bias ? bias[n + 3] : 0.0f;
+  const float c0 = bias ? bias[n] : 0.0f, c1 = bias ? bias[n + 1] : 0.0f;
+  const float c2 = bias ? bias[n + 2] : 0.0f, c3 = bias ? bias[n + 3] : 0.0f;
 #pragma unroll
   for (int r = 0; r < RR; ++r) {
     const int m = m0 + r;
@@ -1766,12 +1803,53 @@ __global__ __launch_bounds__(256) void splitk_reduce4_kernel(const float *__rest
     const float s = rscale ? rscale[m] : 1.0f;
     if (__builtin_isnan(s)) continue;  // the pre-pass wrote this row's IEEE outputs
     f4 o;
-    o.x = __builtin_fmaf(acc[r].x, s, b0);
-    o.y = __builtin_fmaf(acc[r].y, s, b1);
-    o.z = __builtin_fmaf(acc[r].z, s, b2);
-    o.w = __builtin_fmaf(acc[r].w, s, b3);
+    o.x = __builtin_fmaf(acc[r].x, s, c0);
+    o.y = __builtin_fmaf(acc[r].y, s, c1);
+    o.z = __builtin_fmaf(acc[r].z, s, c2);
+    o.w = __builtin_fmaf(acc[r].w, s, c3);
     *reinterpret_cast<f4 *>(Y + (size_t)m * N + n) = o;
   }
+}
+
+// Reduces the partials of matrices with more than one slice: together where
+// every one has whole 16-byte pieces, else one by one.
+static hipError_t launch_splitk_reduce(const ReduceMat *m, int count, int64_t M, const float *rscale, hipStream_t s) {
+  constexpr int RR = kReduceRows;
+  const bool rows_fit = (M + RR - 1) / RR <= 65535;
+  ReduceMats rm{};
+  int c = 0, bx = 0, kmax = 0;
+  for (int i = 0; i < count; ++i) {
+    if (m[i].ks <= 1) continue;
+    if (rows_fit && m[i].n % 4 == 0 && (reinterpret_cast<uintptr_t>(m[i].y) & 15u) == 0) {
+      rm.mat[c] = m[i];
+      rm.mat[c++].bx0 = bx;
+      bx += (m[i].n + 1023) / 1024;
+      kmax = std::max(kmax, m[i].ks);
+      continue;
+    }
+    const dim3 rgrid((unsigned)((m[i].n + 255) / 256), (unsigned)std::min<int64_t>(M, 65535));
+    const int ks = m[i].ks;
+    if (ks <= 2) hipLaunchKernelGGL(splitk_reduce_kernel<2>, rgrid, dim3(256), 0, s, m[i].part, ks, (int)M, m[i].n, rscale, m[i].bias, m[i].y);
+    else if (ks <= 4) hipLaunchKernelGGL(splitk_reduce_kernel<4>, rgrid, dim3(256), 0, s, m[i].part, ks, (int)M, m[i].n, rscale, m[i].bias, m[i].y);
+    else hipLaunchKernelGGL(splitk_reduce_kernel<8>, rgrid, dim3(256), 0, s, m[i].part, ks, (int)M, m[i].n, rscale, m[i].bias, m[i].y);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  if (c == 0) return hipSuccess;
+  for (int i = c; i < kPrefillMats; ++i) rm.mat[i].bx0 = INT32_MAX;
+  const dim3 g4((unsigned)bx, (unsigned)((M + RR - 1) / RR));
+#define OKQ_REDUCE(KB_)                                                                                              \
+  if (c == 1) hipLaunchKernelGGL((splitk_reduce4_kernel<KB_, RR, true>), g4, dim3(256), 0, s, rm, (int)M, rscale);  \
+  else hipLaunchKernelGGL((splitk_reduce4_kernel<KB_, RR, false>), g4, dim3(256), 0, s, rm, (int)M, rscale)
+  if (kmax <= 2) {
+    OKQ_REDUCE(2);
+  } else if (kmax <= 4) {
+    OKQ_REDUCE(4);
+  } else {
+    OKQ_REDUCE(8);
+  }
+#undef OKQ_REDUCE
+  return hipGetLastError();
 }
 
 // The decode-batch kernel's partials [ksplit][M][ntiles * 16] over the
@@ -1873,6 +1951,30 @@ bool gemm_supported(int type, int64_t M, int64_t K, int64_t N) {
          a_bytes < (int64_t)UINT32_MAX && w_bytes < (int64_t)UINT32_MAX;
 }
 
+static size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
+
+// K slices of gemm_f32_*_kernel for one matrix: the split of least estimated
+// time.  A round of workgroups (one per CU) takes ~7 us (Q4_K) per
+// super-block of its slice and ~5 us around its loop; the partials are
+// written and read once at ~4 TB/s, and their reduction is one more launch.
+static int64_t f32_split(int type, int64_t M, int64_t N, int64_t K, int cu_count) {
+  const double us_sb = (type == kQ6_K ? 10.0 : type == kQ8_0 ? 8.5 : 7.0) *
+                       (0.2 + 0.2 * gemm_f32_blocks(M));
+  const int64_t nsb = K / 256, tiles = gemm_f32_tiles(M, N), cus = cu_count;
+  int64_t best = 1;
+  double least = 0.0;
+  // (Q6_K in slices of one super-block: 1.80e-7 from float64, of two 1.73e-7)
+  const int64_t most = std::min<int64_t>(16, type == kQ6_K ? std::max<int64_t>(1, nsb / 2) : nsb);
+  for (int64_t ks = 1; ks <= most; ++ks) {
+    const double bytes = 4.0 * (double)M * (double)N * (double)(2 * ks + 1);
+    if (ks > 1 && bytes > (double)UINT32_MAX) break;  // the reduction's 32-bit offsets, with room
+    const double us = (double)((tiles * ks + cus - 1) / cus) * (us_sb * (double)((nsb + ks - 1) / ks) + 5.0) +
+                      (ks > 1 ? 3.0 + bytes / 4e6 : 0.0);
+    if (ks == 1 || us < least) best = ks, least = us;
+  }
+  return best;
+}
+
 GemmPlan gemm_plan(int type, int64_t M, int64_t N, int64_t K, bool x_is_bf16, int cu_count) {
   GemmPlan p{};
   p.kwaves = 1;
@@ -1951,7 +2053,11 @@ GemmPlan gemm_plan(int type, int64_t M, int64_t N, int64_t K, bool x_is_bf16, in
       const int64_t jobs = t6 * q6_ks, rounds = (jobs + cus - 1) / cus;
       q6_wide = jobs * 4 >= rounds * cus * 3;
     }
-    if (x_is_bf16 && type == kQ8_0) {
+    if (!x_is_bf16) {
+      p.bm = 128;
+      p.wide = 5;
+      ks = f32_split(type, M, N, K, cu_count);
+    } else if (type == kQ8_0) {
       // gemm_q8_kernel (bf16 activations straight from x: no pre-pass).  The
       // 8-wave 128 x 256 tiles (one workgroup per CU) while they fill at
       // least 3/4 of their rounds of CUs (M=2048 4096 x 4096: 1 round);
@@ -2002,7 +2108,7 @@ GemmPlan gemm_plan(int type, int64_t M, int64_t N, int64_t K, bool x_is_bf16, in
     }
   }
   p.ksplit = (int)std::max<int64_t>(1, ks);
-  auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
+  auto up = up256;
   if (p.bm == kDecRows) {  // the decode-batch kernel needs only the split-K partials (whole 16-column tiles)
     p.off_lo = p.off_sums = p.off_rscale = p.off_part = 0;
     p.workspace = p.ksplit > 1 ? up((size_t)p.ksplit * M * ((N + 15) / 16 * 16) * sizeof(float)) : 0;
@@ -2019,8 +2125,28 @@ GemmPlan gemm_plan(int type, int64_t M, int64_t N, int64_t K, bool x_is_bf16, in
   p.off_sums = p.off_lo + (x_is_bf16 ? 0 : up(plane));
   p.off_rscale = p.off_sums + up(sums);
   p.off_part = p.off_rscale + up((size_t)M * sizeof(float));
-  p.workspace = p.off_part + (p.ksplit > 1 ? up((size_t)p.ksplit * M * N * sizeof(float)) : 0);
+  auto parts = [&](int k) { return k > 1 ? up((size_t)k * M * N * sizeof(float)) : (size_t)0; };
+  // a call whose planes fit the allocation-free entry point's scratch stays
+  // within it (one dispatch for both entry points: the same bits)
+  if (p.wide == 5 && p.off_part <= kScratchBytes)
+    while (p.ksplit > 1 && p.off_part + parts(p.ksplit) > kScratchBytes) --p.ksplit;
+  p.workspace = p.off_part + parts(p.ksplit);
   return p;
+}
+
+PrefillPlan prefill_plan(int64_t M, int64_t K, int count, const int *types, const int64_t *N, int cu_count) {
+  PrefillPlan g{};
+  for (int i = 0; i < count; ++i) {
+    const GemmPlan p = gemm_plan(types[i], M, N[i], K, false, cu_count);
+    g.ksplit[i] = p.ksplit;
+    if (i == 0) {
+      g.base = p;
+      g.workspace = p.off_part;
+    }
+    g.off_part[i] = g.workspace;
+    g.workspace += p.workspace - p.off_part;
+  }
+  return g;
 }
 
 // The decode-batch kernel (it converts the activations itself: no pre-pass)
@@ -2170,8 +2296,8 @@ hipError_t launch_gemm_decode_mixed(const void *x, bool x_is_bf16, int64_t M, in
                        false);
 }
 
-// The tiled kernel over the pre-pass's planes (every format; f32 or bf16).
-static hipError_t launch_gemm_tiled(int type, bool x_is_bf16, _Float16 *xhi, _Float16 *xlo, h2 *xsum, float *rscale,
+// The tiled kernel over the pre-pass's plane (bf16 activations).
+static hipError_t launch_gemm_tiled(int type, _Float16 *xhi, h2 *xsum, float *rscale,
                                     const uint8_t *W, const float *bias, float *y, int64_t M, int64_t N, int64_t K,
                                     const GemmPlan &plan, float *part, hipStream_t s) {
   const int m = (int)M, n = (int)N, k = (int)K, ks = plan.ksplit;
@@ -2180,30 +2306,83 @@ static hipError_t launch_gemm_tiled(int type, bool x_is_bf16, _Float16 *xhi, _Fl
   const int tiles = tiles_m * tiles_n;
   const int per_xcd = (tiles * ks + 7) / 8;
   const dim3 grid((unsigned)(per_xcd * 8)), block((unsigned)(plan.bm * 2));
-#define OKQ_GEMM(BM_, LO_, FMT_)                                                                                   \
-  launch_timed(gemm_kq_kernel<BM_, LO_, FMT_>, grid, block, 0u, s, xhi, xlo, xsum, rscale, W, bias, y, m, n, k,     \
+#define OKQ_GEMM(BM_, FMT_)                                                                                      \
+  launch_timed(gemm_kq_kernel<BM_, false, FMT_>, grid, block, 0u, s, xhi, nullptr, xsum, rscale, W, bias, y, m, n, k, \
                tiles_m, tiles, ks, part)
   if (type == kQ6_K) {
-    if (x_is_bf16) OKQ_GEMM(128, false, kQ6_K);
-    else OKQ_GEMM(128, true, kQ6_K);
+    OKQ_GEMM(128, kQ6_K);
   } else if (type == kQ8_0) {
-    if (x_is_bf16) OKQ_GEMM(128, false, kQ8_0);
-    else OKQ_GEMM(128, true, kQ8_0);
+    OKQ_GEMM(128, kQ8_0);
   } else if (type == kQ5_K) {
-    if (plan.bm == 256) OKQ_GEMM(256, false, kQ5_K);
-    else if (x_is_bf16) OKQ_GEMM(128, false, kQ5_K);
-    else OKQ_GEMM(128, true, kQ5_K);
+    if (plan.bm == 256) OKQ_GEMM(256, kQ5_K);
+    else OKQ_GEMM(128, kQ5_K);
   } else if (plan.bm == 256) {
-    OKQ_GEMM(256, false, kQ4_K);
-  } else if (x_is_bf16) {
-    OKQ_GEMM(128, false, kQ4_K);
+    OKQ_GEMM(256, kQ4_K);
   } else {
-    OKQ_GEMM(128, true, kQ4_K);
+    OKQ_GEMM(128, kQ4_K);
   }
 #undef OKQ_GEMM
   return hipGetLastError();
 }
 
+static PrepIeee prep_ieee(int type, int64_t K, const void *w, int64_t N, const float *bias, float *y) {
+  return PrepIeee{static_cast<const uint8_t *>(w), bias, y, (size_t)(K / 256) * (size_t)sb_bytes_of(type), type, (int)N};
+}
+
+template <bool kF32>
+static hipError_t launch_prep(const void *x, int64_t M, int64_t K, _Float16 *xhi, _Float16 *xlo, h2 *xsum, float *rscale,
+                              const PrepIeees &ieee, hipStream_t s) {
+  // chunks of 8 activations per thread: 2 (K <= 4096), 4, 8 held in registers, longer rows read twice
+  const int64_t per_thread = (K / 8 + 255) / 256;
+#define OKQ_PREP(CH_)                                                                                                 \
+  hipLaunchKernelGGL((gemm_prep_kernel<kF32, CH_>), dim3((unsigned)M), dim3(256), 0, s, x, (int)M, (int)K, xhi, xlo,  \
+                     xsum, rscale, ieee)
+  if (per_thread <= 2) OKQ_PREP(2);
+  else if (per_thread <= 4) OKQ_PREP(4);
+  else if (per_thread <= 8) OKQ_PREP(8);
+  else OKQ_PREP(0);
+#undef OKQ_PREP
+  return hipGetLastError();
+}
+
+hipError_t launch_prefill_multi(const void *x, int64_t M, int64_t K, int count, const int *types, const void *const *w,
+                                const int64_t *N, const float *const *bias, float *const *y, void *workspace,
+                                const PrefillPlan &plan, hipStream_t s) {
+  if (count < 1 || count > kPrefillMats || plan.base.wide != 5) return hipErrorInvalidValue;
+  char *ws = static_cast<char *>(workspace);
+  _Float16 *xhi = reinterpret_cast<_Float16 *>(ws), *xlo = reinterpret_cast<_Float16 *>(ws + plan.base.off_lo);
+  h2 *xsum = reinterpret_cast<h2 *>(ws + plan.base.off_sums);
+  float *rscale = reinterpret_cast<float *>(ws + plan.base.off_rscale);
+  PrepIeees ieee{};
+  ReduceMat red[kPrefillMats];
+  for (int i = 0; i < count; ++i) {
+    const int ks = plan.ksplit[i];
+    if (ks < 1 || (ks > 1 && (int64_t)ks * M * N[i] * 4 > (int64_t)UINT32_MAX)) return hipErrorInvalidValue;
+    ieee.mat[i] = prep_ieee(types[i], K, w[i], N[i], bias[i], y[i]);
+    red[i] = ReduceMat{reinterpret_cast<float *>(ws + plan.off_part[i]), bias[i], y[i], (int)N[i], ks, 0};
+  }
+  ieee.count = count;
+  hipError_t e = launch_prep<true>(x, M, K, xhi, xlo, xsum, rscale, ieee, s);
+  // one launch per format, over its matrices
+  bool done[kPrefillMats] = {};
+  for (int i = 0; i < count && e == hipSuccess; ++i) {
+    if (done[i]) continue;
+    PrefillMats mats{};
+    int c = 0;
+    for (int j = i; j < count; ++j) {
+      if (types[j] != types[i]) continue;
+      done[j] = true;
+      mats.mat[c].w = static_cast<const uint8_t *>(w[j]);
+      mats.mat[c].bias = bias[j];
+      mats.mat[c].y = y[j];
+      mats.mat[c].part = reinterpret_cast<float *>(ws + plan.off_part[j]);
+      mats.mat[c].n = (int)N[j];
+      mats.mat[c++].ksplit = plan.ksplit[j];
+    }
+    e = launch_gemm_f32(types[i], xhi, xlo, xsum, rscale, M, K, mats, c, s);
+  }
+  return e != hipSuccess ? e : launch_splitk_reduce(red, count, M, rscale, s);
+}
 
 hipError_t launch_gemm(int type, const void *x, bool x_is_bf16, int64_t M, int64_t K, const void *w, int64_t N,
                        const float *bias, float *y, void *workspace, const GemmPlan &plan, hipStream_t s) {
@@ -2221,51 +2400,28 @@ hipError_t launch_gemm(int type, const void *x, bool x_is_bf16, int64_t M, int64
                          false);
   }
   float *part = plan.ksplit > 1 ? reinterpret_cast<float *>(ws + plan.off_part) : nullptr;
-  const dim3 rgrid((unsigned)((N + 255) / 256), (unsigned)std::min<int64_t>(M, 65535));
   if (ks > 1 && (int64_t)ks * M * N * 4 > (int64_t)UINT32_MAX) return hipErrorInvalidValue;  // excluded by gemm_plan
-  // the split-K reduction of the partials (rscale: the pre-pass's row scales, or none)
-  auto reduce = [&](const float *rscale) {
-    constexpr int RR = kReduceRows;
-    if (N % 4 == 0 && (reinterpret_cast<uintptr_t>(y) & 15u) == 0 && (M + RR - 1) / RR <= 65535) {
-      const dim3 g4((unsigned)((N + 1023) / 1024), (unsigned)((M + RR - 1) / RR));
-      if (ks <= 2) hipLaunchKernelGGL((splitk_reduce4_kernel<2, RR>), g4, dim3(256), 0, s, part, ks, m, n, rscale, bias, y);
-      else if (ks <= 4) hipLaunchKernelGGL((splitk_reduce4_kernel<4, RR>), g4, dim3(256), 0, s, part, ks, m, n, rscale, bias, y);
-      else hipLaunchKernelGGL((splitk_reduce4_kernel<8, RR>), g4, dim3(256), 0, s, part, ks, m, n, rscale, bias, y);
-      return hipGetLastError();
-    }
-    if (ks <= 2) hipLaunchKernelGGL(splitk_reduce_kernel<2>, rgrid, dim3(256), 0, s, part, ks, m, n, rscale, bias, y);
-    else if (ks <= 4) hipLaunchKernelGGL(splitk_reduce_kernel<4>, rgrid, dim3(256), 0, s, part, ks, m, n, rscale, bias, y);
-    else hipLaunchKernelGGL(splitk_reduce_kernel<8>, rgrid, dim3(256), 0, s, part, ks, m, n, rscale, bias, y);
-    return hipGetLastError();
-  };
+  const ReduceMat red{part, bias, y, n, ks, 0};
+  if (plan.wide == 5) {
+    PrefillPlan g{};
+    g.base = plan;
+    g.ksplit[0] = ks;
+    g.off_part[0] = plan.off_part;
+    return launch_prefill_multi(x, M, K, 1, &type, &w, &N, &bias, &y, workspace, g, s);
+  }
   if (plan.wide == 3) {
     if (!x_is_bf16 || type != kQ8_0) return hipErrorInvalidValue;
     hipError_t e = launch_gemm_q8(x, W, bias, y, M, N, K, ks, plan.kwaves, part, s);
-    return e != hipSuccess || ks == 1 ? e : reduce(nullptr);
+    return e != hipSuccess ? e : launch_splitk_reduce(&red, 1, M, nullptr, s);
   }
+  if (!x_is_bf16) return hipErrorInvalidValue;  // f32 activations: plan.wide == 5
   _Float16 *xhi = reinterpret_cast<_Float16 *>(ws);
-  _Float16 *xlo = x_is_bf16 ? nullptr : reinterpret_cast<_Float16 *>(ws + plan.off_lo);
   h2 *xsum = reinterpret_cast<h2 *>(ws + plan.off_sums);
   float *rscale = reinterpret_cast<float *>(ws + plan.off_rscale);
-  // chunks of 8 activations per thread: 2 (K <= 4096), 4, 8 held in registers, longer rows read twice
-  const int64_t per_thread = (K / 8 + 255) / 256;
-  const PrepIeee ieee{W, bias, y, (size_t)(K / 256) * (size_t)sb_bytes_of(type), type, (int)N};
-#define OKQ_PREP(F32_, CH_)                                                                                       \
-  hipLaunchKernelGGL((gemm_prep_kernel<F32_, CH_>), dim3((unsigned)M), dim3(256), 0, s, x, (int)M, (int)K, xhi, xlo, \
-                     xsum, rscale, ieee)
-#define OKQ_PREP_CH(F32_)                     \
-  if (per_thread <= 2) OKQ_PREP(F32_, 2);     \
-  else if (per_thread <= 4) OKQ_PREP(F32_, 4); \
-  else if (per_thread <= 8) OKQ_PREP(F32_, 8); \
-  else OKQ_PREP(F32_, 0)
-  if (x_is_bf16) {
-    OKQ_PREP_CH(false);
-  } else {
-    OKQ_PREP_CH(true);
-  }
-#undef OKQ_PREP_CH
-#undef OKQ_PREP
-  hipError_t e = hipGetLastError();
+  PrepIeees ieee{};
+  ieee.mat[0] = prep_ieee(type, K, W, N, bias, y);
+  ieee.count = 1;
+  hipError_t e = launch_prep<false>(x, M, K, xhi, nullptr, xsum, rscale, ieee, s);
   if (e != hipSuccess) return e;
   if (plan.wide == 4) {
     e = launch_gemm_q6(xhi, rscale, W, bias, y, M, N, K, ks, part, s);
@@ -2274,9 +2430,9 @@ hipError_t launch_gemm(int type, const void *x, bool x_is_bf16, int64_t M, int64
   } else if (plan.wide) {
     e = launch_gemm_wide(type, xhi, xsum, rscale, W, bias, y, M, N, K, ks, part, s);
   } else {
-    e = launch_gemm_tiled(type, x_is_bf16, xhi, xlo, xsum, rscale, W, bias, y, M, N, K, plan, part, s);
+    e = launch_gemm_tiled(type, xhi, xsum, rscale, W, bias, y, M, N, K, plan, part, s);
   }
-  return e != hipSuccess || ks == 1 ? e : reduce(rscale);
+  return e != hipSuccess ? e : launch_splitk_reduce(&red, 1, M, rscale, s);
 }
 
 }  // namespace okq

@@ -89,9 +89,12 @@ struct GemmPlan {
   int wide;            // weights dequantised in registers (bf16 activations): 1 the wide kernel (Q4_K / Q5_K,
                        // 128 x 256 tiles, one workgroup per CU), 2 the pair kernel (Q4_K / Q5_K, 128 x 128
                        // tiles, two per CU), 3 the Q8_0 kernel (128 x 128 or 128 x 256 tiles),
-                       // 4 the Q6_K kernel (128 x 256 tiles)
+                       // 4 the Q6_K kernel (128 x 256 tiles);
+                       // 5 f32 activations, every format (128 x 256 tiles)
   size_t off_lo, off_sums, off_rscale, off_part, workspace;
 };
+// Size of the allocation-free entry point's static scratch.
+constexpr size_t kScratchBytes = 64u << 20;
 GemmPlan gemm_plan(int type, int64_t M, int64_t N, int64_t K, bool x_is_bf16, int cu_count);
 // `workspace` holds plan.workspace bytes (256-aligned); it is reused by later
 // calls on the stream.
@@ -150,5 +153,39 @@ hipError_t launch_gemm_q6(const _Float16 *xhi, const float *rscale, const void *
 int gemm_q8_tiles(int64_t M, int64_t N, int waves);
 hipError_t launch_gemm_q8(const void *x, const void *w, const float *bias, float *y, int64_t M, int64_t N, int64_t K,
                           int ksplit, int waves, float *part, hipStream_t s);
+
+// f32 activations, every linear format (okq_gemm_f32.hip): the pre-pass's two
+// fp16 planes, 128 x 256 tiles, one 8-wave workgroup per CU; up to
+// kPrefillMats matrices of one format that read the same activations in one
+// launch, each with its own K split into whole super-blocks (ksplit > 1:
+// partials [ksplit][M][n] at part).
+constexpr int kPrefillMats = 4;
+struct PrefillMat {
+  const uint8_t *w;
+  const float *bias;
+  float *y, *part;
+  int n, ksplit;
+  int tiles, px0, pxn;  // set by the launch: tiles, first index and count of the matrix's jobs within an XCD
+};
+struct PrefillMats {
+  PrefillMat mat[kPrefillMats];
+};
+int gemm_f32_blocks(int64_t M);  // 32-row blocks of a tile: 2, 3 or 4
+int gemm_f32_tiles(int64_t M, int64_t N);
+// More than 32 f32 rows through up to kPrefillMats matrices of any linear
+// formats that read them (each gemm_supported): one activation pre-pass, one
+// launch per format, one reduction.  Each matrix keeps gemm_plan's split of
+// its own call, so its outputs are that call's bit for bit.
+struct PrefillPlan {
+  GemmPlan base;  // the planes' layout
+  int ksplit[kPrefillMats];
+  size_t off_part[kPrefillMats], workspace;
+};
+PrefillPlan prefill_plan(int64_t M, int64_t K, int count, const int *types, const int64_t *N, int cu_count);
+hipError_t launch_prefill_multi(const void *x, int64_t M, int64_t K, int count, const int *types, const void *const *w,
+                                const int64_t *N, const float *const *bias, float *const *y, void *workspace,
+                                const PrefillPlan &plan, hipStream_t s);
+hipError_t launch_gemm_f32(int type, const _Float16 *xhi, const _Float16 *xlo, const void *xsum, const float *rscale,
+                           int64_t M, int64_t K, PrefillMats &mats, int count, hipStream_t s);
 
 }  // namespace okq

@@ -305,7 +305,7 @@ bool gemv_serves(uint32_t, int64_t rows, int64_t K, uint64_t w_bytes) {
 // host-side stand-in).  Calls on one device share the array: overlapping calls
 // (several streams or threads at once) race.  Nothing in it needs clearing:
 // every kernel writes the scratch it later reads.
-constexpr size_t kScratchBytes = 64u << 20;
+using okq::kScratchBytes;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 std::mutex g_scratch_mutex;
@@ -580,6 +580,28 @@ okq_status okq_linear_out_by_in_q_bf16(const uint16_t *x, int64_t rows, int64_t 
   return linear_impl(x, true, rows, in_features, w_type, w, w_bytes, out_features, bias, out, stream, Path::Auto);
 }
 
+// More than 32 f32 rows through `count` MFMA-routed matrices (the stream's
+// enqueue lock held): bit for bit each matrix's own call.  Where the shared
+// workspace cannot be had (a capture before any call of this size), the
+// matrices run one by one, each within the workspace of its own call.
+static okq_status prefill_multi(const float *x, int64_t rows, int64_t K, int count, const int *types,
+                                const void *const *w, const int64_t *N, const float *const *bias, float *const *out,
+                                hipStream_t s, int dev, const DevInfo &info) {
+  const okq::PrefillPlan plan = okq::prefill_plan(rows, K, count, types, N, info.cu_count);
+  void *ws = nullptr;
+  if (get_workspace(dev, s, plan.workspace, &ws) == OKQ_OK)
+    return hip_status(okq::launch_prefill_multi(x, rows, K, count, types, w, N, bias, out, ws, plan, s),
+                      "grouped gemm launch");
+  for (int i = 0; i < count; ++i) {
+    const okq::GemmPlan p = okq::gemm_plan(types[i], rows, N[i], K, false, info.cu_count);
+    okq_status st = get_workspace(dev, s, p.workspace, &ws);
+    if (st != OKQ_OK) return st;
+    st = hip_status(okq::launch_gemm(types[i], x, false, rows, K, w[i], N[i], bias[i], out[i], ws, p, s), "gemm launch");
+    if (st != OKQ_OK) return st;
+  }
+  return ok();
+}
+
 // Several validated quantized linears of one format and K that read the same
 // activations x (device f32 [rows][K]); outputs out[i] [rows][N[i]].
 // A matrix that the linear dispatch would not give to the GEMV at this row
@@ -594,7 +616,7 @@ okq_status okq_linear_out_by_in_q_bf16(const uint16_t *x, int64_t rows, int64_t 
 // swiglu_pair (count 2: gate then up of a gated-SiLU MLP): when both take one
 // decode-batch launch that splits K, its reduction also applies the SiLU
 // (out[0] = silu(gate) * up, out[1] = up) and *swiglu_done says so.
-okq_status grouped_linear(const float *x, int64_t rows, int64_t in_features, uint32_t w_type, int count,
+static okq_status grouped_linear(const float *x, int64_t rows, int64_t in_features, uint32_t w_type, int count,
                           const void *const *w, const uint64_t *w_bytes, const int64_t *out_features,
                           const float *const *b, float *const *out, void *stream, int dev, const DevInfo &info,
                           bool swiglu_pair = false, bool *swiglu_done = nullptr) {
@@ -639,6 +661,14 @@ okq_status grouped_linear(const float *x, int64_t rows, int64_t in_features, uin
                     "gemv_multi decode-batch launch");
     if (st != OKQ_OK) return st;
     if (swiglu_done) *swiglu_done = swiglu;
+    grouped = true;
+  }
+  if (mfma > 1 && !grouped) {
+    // prefill: one pre-pass of the shared activations, one launch, one reduction
+    int types[okq::kGemvMaxProblems];
+    for (int i = 0; i < mfma; ++i) types[i] = (int)w_type;
+    st = prefill_multi(x, rows, in_features, mfma, types, mw, mn, mb, mo, s, dev, info);
+    if (st != OKQ_OK) return st;
     grouped = true;
   }
   for (int i = 0; i < mfma && !grouped; ++i) {
@@ -724,6 +754,28 @@ okq_status okq_linear_multi_q(const float *x, int64_t rows, int64_t in_features,
       mtype[mfma] = (int)t;
       midx[mfma++] = i;
       (pass == 0 ? n4 : n6) += 1;
+    }
+  }
+  if (rows > okq::kGemmDecodeRows) {
+    // prefill: the matrices of every format that the MFMA kernels take share
+    // one pre-pass and one reduction
+    const void *mw[okq::kGemvMaxProblems];
+    int64_t mn[okq::kGemvMaxProblems];
+    const float *mb[okq::kGemvMaxProblems];
+    float *mo[okq::kGemvMaxProblems];
+    int types[okq::kGemvMaxProblems], c = 0;
+    for (int i = 0; i < count; ++i) {
+      if (out_features[i] <= 0 || !okq::gemm_supported((int)w_types[i], rows, in_features, out_features[i])) continue;
+      types[c] = (int)w_types[i];
+      mw[c] = w[i];
+      mn[c] = out_features[i];
+      mb[c] = b[i];
+      mo[c++] = out[i];
+      taken[i] = true;
+    }
+    if (c > 0) {
+      st = prefill_multi(x, rows, in_features, c, types, mw, mn, mb, mo, s, dev, info);
+      if (st != OKQ_OK) return st;
     }
   }
   if (rows <= okq::kGemmDecodeRows && n4 > 0 && n6 > 0) {

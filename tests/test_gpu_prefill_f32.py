@@ -1,0 +1,139 @@
+"""GPU parity of prefill with f32 activations (more than 32 rows, every linear
+format) and of several matrices sharing one call (needs an MI355X).
+
+Bars: outputs against float64 on the oracle's dequantised weights; the shared
+calls bit for bit against each matrix's own call.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+TYPES = [O.Q4_K, O.Q5_K, O.Q6_K, O.Q8_0]
+
+
+@pytest.fixture(scope="module")
+def torch():
+    import torch as _t
+    if not _t.cuda.is_available():
+        pytest.skip("no GPU")
+    return _t
+
+
+@pytest.fixture(scope="module")
+def okq(torch):
+    from ocelotl_amd import okq as _okq
+    _okq.call("okq_init", 0)
+    return _okq
+
+
+@pytest.fixture(scope="module")
+def orc():
+    return O.Oracle()
+
+
+def _dev(torch, a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def _linear(torch, okq, t, xd, rows, k, wd, n, bd=None, entry="okq_linear_out_by_in_q", stream=None):
+    out = torch.full((rows * n,), float("nan"), dtype=torch.float32, device="cuda")
+    okq.call(entry, xd.data_ptr(), rows, k, t, wd.data_ptr(), wd.numel(), n, None if bd is None else bd.data_ptr(),
+             out.data_ptr(), torch.cuda.current_stream().cuda_stream if stream is None else stream)
+    return out
+
+
+@pytest.mark.parametrize("t", TYPES)
+@pytest.mark.parametrize("rows,k,n", [
+    (33, 256, 40),      # one super-block, the 64-row tile mostly padding
+    (64, 768, 255),     # a full 64-row tile, an odd number of super-blocks
+    (65, 2304, 257),    # 96-row tiles, two column tiles, split K
+    (97, 512, 512), (128, 4096, 300), (129, 1280, 96), (333, 1024, 520),
+    (300, 8192, 4096),  # unsplit or long slices: Q8_0's sums wait in the output or the partials
+    (1100, 7424, 4100),
+])
+def test_f32_prefill_matches_float64(torch, okq, orc, t, rows, k, n):
+    """Every product is exact but for the activations' hi + lo planes (2^-22)
+    and, in Q6_K, the dropped lo * remainder (2^-22); f32 sums of up to 3 K / 16
+    MFMA accumulations round at random: 2^-20 of sum |x| max |w| bounds them
+    with room (one wrong product of K would be 1 / K)."""
+    print(f"[gpu] f32 prefill type={t} rows={rows} K={k} N={n}", flush=True)
+    wq = orc.quantize(t, orc.normal(9000 + t + k, n * k, 0.02))
+    x = orc.normal(9001 + rows, rows * k, 1.0).reshape(rows, k)
+    x[:, :3] *= 100.0
+    x[rows // 2] *= np.float32(2.0 ** 30)
+    bias = orc.normal(9002, n, 0.1)
+    xd, wd, bd = _dev(torch, x), _dev(torch, wq), _dev(torch, bias)
+    out = _linear(torch, okq, t, xd, rows, k, wd, n, bd)
+    torch.cuda.synchronize()
+    w = _dev(torch, orc.dequantize(t, wq, n * k)).view(n, k).double()
+    want = xd.double() @ w.t() + bd.double()
+    bound = 2.0 ** -20 * xd.double().abs().sum(1, keepdim=True) * 2 * w.abs().amax(1) + 2.0 ** -22 * want.abs()
+    err = (out.view(rows, n).double() - want).abs()
+    assert bool((err <= bound).all()), float((err / bound).max())
+
+
+@pytest.mark.parametrize("types,rows,k,ns", [
+    ([O.Q4_K, O.Q4_K, O.Q6_K], 70, 4096, [1024, 256, 256]),
+    ([O.Q8_0, O.Q8_0, O.Q8_0], 333, 2048, [2048, 512, 300]),
+    ([O.Q5_K, O.Q6_K, O.Q5_K, O.Q8_0], 40, 768, [33, 300, 512, 17]),
+])
+def test_f32_prefill_matrices_share_a_call_bit_for_bit(torch, okq, orc, types, rows, k, ns):
+    """okq_linear_multi_q above 32 rows: one pre-pass, one launch per format,
+    one reduction; every output is its own call's, also in rows with an
+    infinity or a NaN."""
+    print(f"[gpu] f32 prefill shared types={types} rows={rows} K={k} N={ns}", flush=True)
+    x = orc.normal(9100 + rows, rows * k, 1.0).reshape(rows, k)
+    x[3, 5], x[rows - 1, 7], x[rows - 1, 9] = np.inf, np.nan, -np.inf
+    xd = _dev(torch, x)
+    wds = [_dev(torch, orc.quantize(t, orc.normal(9110 + i, n * k, 0.02))) for i, (t, n) in enumerate(zip(types, ns))]
+    bds = [_dev(torch, orc.normal(9120 + i, n, 0.1)) if i != 1 else None for i, n in enumerate(ns)]
+    outs = [torch.full((rows * n,), 7.0, dtype=torch.float32, device="cuda") for n in ns]
+    arr = lambda ty, vals: (ty * len(ns))(*vals)
+    args = (xd.data_ptr(), rows, k, len(ns), arr(ctypes.c_uint32, types), arr(ctypes.c_void_p, [w.data_ptr() for w in wds]),
+            arr(ctypes.c_uint64, [w.numel() for w in wds]), arr(ctypes.c_int64, ns),
+            arr(ctypes.c_void_p, [None if b is None else b.data_ptr() for b in bds]),
+            arr(ctypes.c_void_p, [o.data_ptr() for o in outs]))
+    okq.call("okq_linear_multi_q", *args, torch.cuda.current_stream().cuda_stream)
+    single = [_linear(torch, okq, t, xd, rows, k, w, n, b) for t, w, n, b in zip(types, wds, ns, bds)]
+    torch.cuda.synchronize()
+    for o, s in zip(outs, single):
+        a, b = o.cpu().numpy(), s.cpu().numpy()
+        assert ((a.view(np.uint32) == b.view(np.uint32)) | (np.isnan(a) & np.isnan(b))).all()
+        assert np.isnan(a.reshape(rows, -1)[rows - 1]).all() and not np.isfinite(a.reshape(rows, -1)[3]).any()
+    # under capture on a stream that has only served single calls: the same bits
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for t, w, n, b in zip(types, wds, ns, bds):
+            _linear(torch, okq, t, xd, rows, k, w, n, b, stream=side.cuda_stream)
+    side.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        okq.call("okq_linear_multi_q", *args, side.cuda_stream)
+    for _ in range(3):
+        for o in outs:
+            o.fill_(7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        for o, s in zip(outs, single):
+            a, b = o.cpu().numpy(), s.cpu().numpy()
+            assert ((a.view(np.uint32) == b.view(np.uint32)) | (np.isnan(a) & np.isnan(b))).all()
+
+
+def test_f32_prefill_near_the_static_scratch(torch, okq, orc):
+    """2800 rows of 4096: the two planes take 46 of the 64 MiB of the
+    allocation-free entry point, so the K split that would fill the CUs is cut
+    to fit; both entry points take the same split."""
+    t, rows, k, n = O.Q4_K, 2800, 4096, 512
+    print(f"[gpu] f32 prefill scratch rows={rows} K={k} N={n}", flush=True)
+    wd = _dev(torch, orc.quantize(t, orc.normal(9200, n * k, 0.02)))
+    xd = torch.randn(rows * k, generator=torch.Generator().manual_seed(9201)).cuda()
+    a = _linear(torch, okq, t, xd, rows, k, wd, n, entry="okq_linear_out_by_in_q_noalloc")
+    b = _linear(torch, okq, t, xd, rows, k, wd, n)
+    torch.cuda.synchronize()
+    assert (a.cpu().numpy().view(np.uint32) == b.cpu().numpy().view(np.uint32)).all()
