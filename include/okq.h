@@ -249,9 +249,10 @@ okq_status okq_rmsnorm_linear_q_multi(const float *x, int64_t rows, int64_t hidd
  * row_bytes(intermediate)); gate_buf, up_buf [rows, intermediate] caller-owned
  * scratch; out [rows, hidden].  Device buffers, x/gate_buf/up_buf 16-byte
  * aligned.  Decode-sized rows (rows <= 8) run gate+up as one grouped GEMV
- * when they share a format.  A single row folds silu(gate) * up into the down
- * GEMV's prologue whenever the down weight takes the streaming GEMV (gate_buf
- * then holds gate(x)); otherwise silu(gate(x)) * up(x) is left in gate_buf,
+ * when they share a format.  A single row computes silu(gate) * up on the way
+ * (in the gate+up launch where its rows go in pairs, through a per-stream
+ * workspace, else in the down GEMV's prologue) whenever the down weight takes
+ * the streaming GEMV (gate_buf then holds gate(x)); otherwise silu(gate(x)) * up(x) is left in gate_buf,
  * as the reference does (when gate and up share one decode-batch launch that
  * splits K, by its reduction: no separate pass over the intermediate).  up_buf always holds up(x).  Treat both as scratch.  Zero rows, hidden or
  * intermediate are errors (mlp.rs:151-165). */

@@ -506,6 +506,12 @@ struct GemvMore {
   int start[kGemvMaxProblems - 1];
 };
 
+// silu(g) * u in the reference's order (crates/kernels/src/mlp.rs:77-88).
+__device__ __forceinline__ float silu_times(float g, float u) {
+  const float sig = 1.0f / (1.0f + expf(-g));
+  return (g * sig) * u;
+}
+
 constexpr int kMaxXV = 4;        // float4s of x per thread, one-row launches (K <= 4 * 4 * 1024)
 constexpr int kMaxXVRows = 8;    // per thread and row, multi-row launches (K <= 8 * 4 * 512)
 constexpr int kPartChunk = 32;   // steps whose team partial sums wait in LDS
@@ -550,11 +556,23 @@ constexpr int gemv_max_threads() {
 // step-major order by an LDS counter, so the waves that the SIMD arbiters
 // favour take more rows and a workgroup's waves finish together.  Results
 // are the same bits as the static order's (every row is one wave's work).
-template <class F, int D, int XV, bool kMulti, int kPro, int R, bool kDyn>
-__global__ __launch_bounds__(gemv_max_threads<R>()) void gemv_kernel(
-    const uint8_t *__restrict__ W, uint32_t w_bytes, const float *__restrict__ x, const float *__restrict__ bias,
-    float *__restrict__ y, int N, int K, int T, int G, GemvMore M, GemvPro P, int nrows) {
+//
+// kPair (two matrices of equal rows, gate then up; dynamic rows of both in a
+// ring of two): a "row" is row i of both matrices, ring slot 0 holding the
+// gate's and slot 1 the up's, so one wave has both sums and writes, besides
+// them, silu(gate) * up to P.h.  The down projection then reads finished
+// activations: as its prologue, the SiLU of all 14336 of them in every
+// workgroup, made a Q6_K down launch 17.4 us where it is 14.1 without, and the
+// pairs cost gate + up 0.4 us.
+//
+// bi, nb: the workgroup's index among those of the launch that stream these
+// matrices, and their number.
+template <class F, int D, int XV, bool kMulti, int kPro, int R, bool kDyn, bool kPair>
+__device__ __forceinline__ void gemv_body(const uint8_t *__restrict__ W, uint32_t w_bytes, const float *__restrict__ x,
+                                          const float *__restrict__ bias, float *__restrict__ y, int N, int K, int T,
+                                          int G, const GemvMore &M, const GemvPro &P, int nrows, int bi, int nb) {
   static_assert(kPro == kProNone || R == 1, "the neighbour prologues take one activation row");
+  static_assert(!kPair || (kDyn && kMulti && R == 1 && D == 2), "pairs: dynamic rows, one of each matrix in the ring");
   // kDyn launches have T == 1 (one wave per row), checked by the launcher
   __shared__ unsigned next_row;  // kDyn: the workgroup's next row index
   __shared__ unsigned qflags[16];  // per wave: the run status bits of its lanes
@@ -573,11 +591,11 @@ __global__ __launch_bounds__(gemv_max_threads<R>()) void gemv_kernel(
   const uint32_t rb = (uint32_t)F::row_bytes(K);
   const uint32_t uoff = active ? F::unit_off(u) : 0u;
   const uint32_t idle_mask = active ? 0u : 0xFFFFFFFFu;  // kDyn
-  const int window = (int)gridDim.x * G;         // rows per step
+  const int window = nb * G;                     // rows per step
   const int steps = (N + window - 1) / window;  // grid-uniform
   const int end = N;
   float inv_rms = 0.0f;  // kProRms: 1 / rms of the row (the IEEE path reapplies it)
-  auto row_of = [&](int step) { return step * window + (int)blockIdx.x * G + g; };
+  auto row_of = [&](int step) { return step * window + bi * G + g; };
   // Matrix selection: single-matrix launches (kMulti = false) never touch M;
   // in multi-matrix launches a row finds its matrix from the three row
   // boundaries and reads that matrix's record with scalar loads at a
@@ -617,6 +635,12 @@ __global__ __launch_bounds__(gemv_max_threads<R>()) void gemv_kernel(
     }
     F::load(Rg, rsrc(p), off, lane);
   };
+  // kPair: row `row` of matrix j
+  auto wload_pair = [&](typename F::Regs &Rg, int row, int j) {
+    const uint32_t endb = bytes_of(j);
+    const uint32_t in = row < end ? (uint32_t)row * rb + uoff : endb;
+    F::load(Rg, rsrc(j), in ^ ((in ^ endb) & idle_mask), lane);
+  };
   // bias values are wave-uniform scalar loads, outside the vector-memory
   // queue that the weight waits count (the dynamic loop reads them through
   // the constant address space: the bias is read-only for the launch, and
@@ -654,19 +678,18 @@ __global__ __launch_bounds__(gemv_max_threads<R>()) void gemv_kernel(
     auto xval = [&](int r, int k) -> float {
       const float v = x[(size_t)r * K + k];
       if constexpr (kPro == kProRms) return v * inv_rms * P.a[k];
-      if constexpr (kPro == kProSwiGLU) {
-        const float sig = 1.0f / (1.0f + expf(-v));
-        return (v * sig) * P.a[k];
-      }
+      if constexpr (kPro == kProSwiGLU) return silu_times(v, P.a[k]);
       return v;
     };
-    for (int st = w; st < steps; st += T) {
+    float gate_sum = 0.0f;  // kPair: T == 1, both passes of a step in one wave
+    for (int st2 = w; st2 < (kPair ? 2 * steps : steps); st2 += T) {
+      const int st = kPair ? st2 >> 1 : st2;
       const int row = row_of(st);
       if (row >= end) break;
-      const int p = prob(row);
-      const uint32_t roff = (uint32_t)(row - first_row(p)) * rb;
+      const int p = kPair ? st2 & 1 : prob(row);
+      const uint32_t roff = (uint32_t)(row - (kPair ? 0 : first_row(p))) * rb;
       const uint8_t *rowp = wbase_of(p) + roff;
-      const float bv = bload(row);
+      const float bv = kPair ? 0.0f : bload(row);
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         if (r >= nrows) break;
@@ -690,7 +713,13 @@ __global__ __launch_bounds__(gemv_max_threads<R>()) void gemv_kernel(
           const float sum = wave_sum(acc);
           tot = T == 1 ? sum : tot + sum;
         }
-        if (lane == 0) store(row, r, tot + bv);
+        if constexpr (kPair) {
+          if (lane == 0) y_of(p)[row] = tot;
+          if (p == 1 && lane == 0) P.h[row] = silu_times(gate_sum, tot);
+          gate_sum = tot;
+        } else {
+          if (lane == 0) store(row, r, tot + bv);
+        }
       }
     }
   };
@@ -728,8 +757,12 @@ __global__ __launch_bounds__(gemv_max_threads<R>()) void gemv_kernel(
   float bs[D];
 #pragma unroll
   for (int j = 0; j < 1; ++j) {
-    wload(S[j], row_of(j));
-    bs[j] = bload(row_of(j));
+    if constexpr (kPair) {
+      wload_pair(S[j], row_of(0), j);
+    } else {
+      wload(S[j], row_of(j));
+      bs[j] = bload(row_of(j));
+    }
   }
 
   // 3. (optional neighbour transform, then) quantise x into LDS while the
@@ -759,11 +792,7 @@ __global__ __launch_bounds__(gemv_max_threads<R>()) void gemv_kernel(
       xv[0][i].w = as_u32(as_f32(xv[0][i].w) * inv * as_f32(av[i].w));
     }
   } else if constexpr (kPro == kProSwiGLU) {
-    auto gate = [](uint32_t gb, uint32_t ub) {
-      const float gv = as_f32(gb);
-      const float sig = 1.0f / (1.0f + expf(-gv));
-      return as_u32((gv * sig) * as_f32(ub));
-    };
+    auto gate = [](uint32_t gb, uint32_t ub) { return as_u32(silu_times(as_f32(gb), as_f32(ub))); };
 #pragma unroll
     for (int i = 0; i < XV; ++i) {
       xv[0][i].x = gate(xv[0][i].x, av[i].x);
@@ -829,6 +858,38 @@ __global__ __launch_bounds__(gemv_max_threads<R>()) void gemv_kernel(
       }
     };
 
+    if constexpr (kPair) {
+      // slot 0 the gate's row, slot 1 the up's; each is refilled with the
+      // next pair's as soon as it is consumed, the pair taken at slot 0
+      int row = row_of(0);
+      float gs = 0.0f;
+      auto sum_of = [&](int j) { return wave_sum(F::compute(S[j], xreg[0], xlo[0], wide_rows & 1u, lane)); };
+      auto put = [&](float us) {  // lane 0 alone, as below
+        if (lane == 0 && row < end) {
+          M.mat[0].y[row] = gs;
+          M.mat[1].y[row] = us;
+          P.h[row] = silu_times(gs, us);
+        }
+      };
+      for (;;) {
+        unsigned c = 0;
+        if (lane == 0) {
+          const uint32_t addr = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned *)&next_row;
+          asm volatile("ds_add_rtn_u32 %0, %1, %2\n\ts_waitcnt lgkmcnt(0)" : "=v"(c) : "v"(addr), "v"(1u));
+        }
+        gs = sum_of(0);
+        c = (unsigned)__builtin_amdgcn_readfirstlane((int)c);
+        const int cs = (int)(c / (unsigned)G);
+        const int nrow = (cs * nb + bi) * G + (int)(c - (unsigned)cs * (unsigned)G);
+        if (nrow >= end) break;
+        wload_pair(S[0], nrow, 0);
+        put(sum_of(1));
+        wload_pair(S[1], nrow, 1);
+        row = nrow;
+      }
+      put(sum_of(1));
+      return;
+    }
     if constexpr (kDyn) {
       // Ring slot j holds row ring_row[j]; a wave's rows increase in slot
       // order.  Idle lanes read zeros and hold zero activations, so the compute
@@ -856,7 +917,6 @@ __global__ __launch_bounds__(gemv_max_threads<R>()) void gemv_kernel(
             if (r < nrows) store(row, r, sum[r] + bs[j]);
         }
       };
-      const int nb = (int)gridDim.x, bi = (int)blockIdx.x;
       while (ring_row[D - 1] < end) {
   #pragma unroll
         for (int j = 0; j < D; ++j) {
@@ -917,14 +977,18 @@ __global__ __launch_bounds__(gemv_max_threads<R>()) void gemv_kernel(
   for (int b = 0; b < 2 * R; ++b)
     if (__ballot((qst >> b) & 1u) != 0ull) wst |= 1u << b;
   if (lane == 0) qflags[wave] = wst;
-  if (kDyn && tid == 0) next_row = (unsigned)(D * G);
+  if (kDyn && tid == 0) next_row = (unsigned)((kPair ? 1 : D) * G);
   __syncthreads();
   if (g >= G) return;  // helper wave (T == 1: no barriers follow)
   {
 #pragma unroll
     for (int j = 1; j < D; ++j) {
-      wload(S[j], row_of(j));
-      bs[j] = bload(row_of(j));
+      if constexpr (kPair) {
+        wload_pair(S[j], row_of(0), j);
+      } else {
+        wload(S[j], row_of(j));
+        bs[j] = bload(row_of(j));
+      }
     }
   }
   unsigned st_all = 0u;
@@ -945,6 +1009,33 @@ __global__ __launch_bounds__(gemv_max_threads<R>()) void gemv_kernel(
     return;
   }
   stream_rows(wide);
+}
+
+template <class F, int D, int XV, bool kMulti, int kPro, int R, bool kDyn, bool kPair>
+__global__ __launch_bounds__(gemv_max_threads<R>()) void gemv_kernel(
+    const uint8_t *__restrict__ W, uint32_t w_bytes, const float *__restrict__ x, const float *__restrict__ bias,
+    float *__restrict__ y, int N, int K, int T, int G, GemvMore M, GemvPro P, int nrows) {
+  gemv_body<F, D, XV, kMulti, kPro, R, kDyn, kPair>(W, w_bytes, x, bias, y, N, K, T, G, M, P, nrows, (int)blockIdx.x,
+                                                    (int)gridDim.x);
+}
+
+// Matrices of two formats against one activation row in one launch (a
+// Q4_K_M layer's q, k and v): workgroups below nb1 stream the first format's
+// rows (N1, G1 teams each), the others the second's.  Each format's
+// workgroups are shared out by weight bytes, so both streams end together.
+// 5120 x 4096 Q4_K and 1024 x 4096 Q6_K: two launches 6.2 + 4.6 us (the second
+// has 3 MB to read, its cost is the launch), this one 7.4 us.
+template <class F1, class F2, int XV>
+__global__ __launch_bounds__(1024) void gemv_mixed_kernel(const float *__restrict__ x, int K, int T, int N1, int G1,
+                                                          int nb1, GemvMore M1, int N2, int G2, GemvMore M2) {
+  const GemvPro none{};
+  const int b = (int)blockIdx.x;
+  if (b < nb1)
+    gemv_body<F1, 1, XV, true, kProNone, 1, false, false>(nullptr, 0u, x, nullptr, nullptr, N1, K, T, G1, M1, none, 1, b,
+                                                          nb1);
+  else
+    gemv_body<F2, 1, XV, true, kProNone, 1, false, false>(nullptr, 0u, x, nullptr, nullptr, N2, K, T, G2, M2, none, 1,
+                                                          b - nb1, (int)gridDim.x - nb1);
 }
 
 // ---------------------------------------------------------------------------
@@ -992,14 +1083,21 @@ struct GemvLaunch {
 template <class F, int D, int XV, bool kMulti, int kPro, int R>
 void launch_kernel(dim3 grid, dim3 block, size_t lds, hipStream_t s, const GemvLaunch &L, const float *x, int k,
                    int T, int G) {
-  if constexpr (XV <= 2 && D == F::kMaxDepth) {
-    if (L.dyn && T == 1) {
-      launch_timed(gemv_kernel<F, D, XV, kMulti, kPro, R, true>, grid, block, (unsigned)lds, s, L.w, L.bytes, x,
+  if constexpr (XV <= 2 && D == 2 && kMulti && kPro == kProNone && R == 1) {
+    if (L.P.h) {
+      launch_timed(gemv_kernel<F, D, XV, kMulti, kPro, R, true, true>, grid, block, (unsigned)lds, s, L.w, L.bytes, x,
                    L.bias, L.y, L.rows, k, T, G, L.M, L.P, L.nrows);
       return;
     }
   }
-  launch_timed(gemv_kernel<F, D, XV, kMulti, kPro, R, false>, grid, block, (unsigned)lds, s, L.w, L.bytes, x, L.bias,
+  if constexpr (XV <= 2 && D == F::kMaxDepth) {
+    if (L.dyn && T == 1) {
+      launch_timed(gemv_kernel<F, D, XV, kMulti, kPro, R, true, false>, grid, block, (unsigned)lds, s, L.w, L.bytes, x,
+                   L.bias, L.y, L.rows, k, T, G, L.M, L.P, L.nrows);
+      return;
+    }
+  }
+  launch_timed(gemv_kernel<F, D, XV, kMulti, kPro, R, false, false>, grid, block, (unsigned)lds, s, L.w, L.bytes, x, L.bias,
                L.y, L.rows, k, T, G, L.M, L.P, L.nrows);
 }
 
@@ -1133,6 +1231,9 @@ hipError_t launch_gemv_multi(int type, const float *x, int64_t K, int64_t rows, 
   if (type != kQ4_K && type != kQ5_K && type != kQ6_K && type != kQ8_0) return hipErrorInvalidValue;
   if (count < 1 || count > kGemvMaxProblems) return hipErrorInvalidValue;
   if (pro.kind != kProNone && rows != 1) return hipErrorNotSupported;  // prologues run one row at a time
+  if (pro.h && (pro.kind != kProNone || rows != 1 || count != 2 || N[0] != N[1] || bias[0] || bias[1] ||
+                !gemv_pairs(type, K, w[0], w[1], N[0], cu_count)))
+    return hipErrorInvalidValue;
   GemvLaunch P{};
   P.P = pro;
   int64_t total = 0;
@@ -1177,7 +1278,7 @@ hipError_t launch_gemv_multi(int type, const float *x, int64_t K, int64_t rows, 
       P.M.start[i - 1] = INT32_MAX;
     }
   }
-  P.rows = (int)total;
+  P.rows = (int)(pro.h ? N[0] : total);  // pairs: row i of both matrices
   if (total == 0) return hipSuccess;
   // up to kMaxRowsPerLaunch activation rows per pass over the weights, as
   // many as the LDS holds: R rows of XRecs plus the teams' partial sums
@@ -1196,6 +1297,81 @@ hipError_t launch_gemv_multi(int type, const float *x, int64_t K, int64_t rows, 
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
+}
+
+// Gate and up rows in pairs: one wave per row, the two-row ring (its formats
+// are those of at least two rows in flight), and more than two steps, so that
+// the rows are handed out dynamically.
+bool gemv_pairs(int type, int64_t K, const void *gate, const void *up, int64_t N, int cu_count) {
+  return (type == kQ4_K || type == kQ5_K || type == kQ8_0) && K <= 4096 && N > 2 * 16 * (int64_t)cu_count &&
+         N < (int64_t)INT32_MAX / 2 && fast_ok(type, K, gate, N) && fast_ok(type, K, up, N);
+}
+
+bool gemv_mixes(int64_t K, int count, const int *types, const void *const *w, const int64_t *N) {
+  int64_t n4 = 0, n6 = 0;
+  for (int i = 0; i < count; ++i) {
+    if (N[i] < 1 || (types[i] != kQ4_K && types[i] != kQ6_K) || !fast_ok(types[i], K, w[i], N[i])) return false;
+    (types[i] == kQ4_K ? n4 : n6) += N[i];
+  }
+  return n4 > 0 && n6 > 0 && n4 < (int64_t)INT32_MAX && n6 < (int64_t)INT32_MAX;
+}
+
+hipError_t launch_gemv_mixed(const float *x, int64_t K, int count, const int *types, const void *const *w,
+                             const int64_t *N, const float *const *bias, float *const *y, int cu_count,
+                             hipStream_t s) {
+  if (!gemv_mixes(K, count, types, w, N) || cu_count < 2) return hipErrorInvalidValue;
+  GemvMore M[2] = {};
+  int64_t rows[2] = {0, 0}, bytes[2] = {0, 0};
+  for (int f = 0; f < 2; ++f) {
+    const int t = f == 0 ? kQ4_K : kQ6_K;
+    int c = 0;
+    for (int i = 0; i < count; ++i) {
+      if (types[i] != t) continue;
+      const size_t b = (size_t)N[i] * row_bytes_of(t, K);
+      M[f].mat[c] = GemvMat{static_cast<const uint8_t *>(w[i]), bias[i], y[i], (uint32_t)b, (int)rows[f], (int)N[i], 0};
+      if (c > 0) M[f].start[c - 1] = (int)rows[f];
+      rows[f] += N[i];
+      bytes[f] += (int64_t)b;
+      ++c;
+    }
+    for (; c < kGemvMaxProblems; ++c) {
+      M[f].mat[c] = GemvMat{nullptr, nullptr, nullptr, 0u, INT32_MAX, 0, 0};
+      if (c > 0) M[f].start[c - 1] = INT32_MAX;
+    }
+  }
+  // workgroups by bytes; per format the fewest teams that finish in as many
+  // steps as the most would (launch_stream's rule)
+  const int U = (int)(K / 64), T = (U + 63) / 64;
+  const int64_t max_g = std::max(1, 16 / T);
+  int64_t nb[2], G[2];
+  nb[0] = std::min<int64_t>(std::max<int64_t>(1, (cu_count * bytes[0] + (bytes[0] + bytes[1]) / 2) / (bytes[0] + bytes[1])),
+                            cu_count - 1);
+  nb[1] = cu_count - nb[0];
+  for (int f = 0; f < 2; ++f) {
+    const int64_t steps = (rows[f] + nb[f] * max_g - 1) / (nb[f] * max_g);
+    G[f] = std::min<int64_t>(max_g, (rows[f] + nb[f] * steps - 1) / (nb[f] * steps));
+    nb[f] = std::min<int64_t>(nb[f], (rows[f] + G[f] * steps - 1) / (G[f] * steps));
+  }
+  const int64_t x_threads = (K / 4 + kMaxXV - 1) / kMaxXV;
+  int64_t g = std::max(G[0], G[1]);
+  if (T > 1) {  // every team joins the barriers: the same number for both formats
+    g = std::max<int64_t>(g, (x_threads + 64 * T - 1) / (64 * T));
+    G[0] = G[1] = g;
+  }
+  int64_t threads = 64 * T * g;
+  if (T == 1) threads = std::min<int64_t>(1024, std::max(threads, (x_threads + 63) / 64 * 64));
+  const int xv = (int)((K / 4 + threads - 1) / threads);
+  if (xv > kMaxXV || threads > 1024) return hipErrorInvalidConfiguration;  // excluded by fast_ok's K bound
+  const size_t lds = (size_t)U * sizeof(XRec) + (T > 1 ? sizeof(float) * kPartChunk * g * T : 0);
+  const dim3 grid((unsigned)(nb[0] + nb[1])), block((unsigned)threads);
+#define OKQ_MIXED(XV_)                                                                                              \
+  launch_timed(gemv_mixed_kernel<FQ4K, FQ6K, XV_>, grid, block, (unsigned)lds, s, x, (int)K, T, (int)rows[0], (int)G[0], \
+               (int)nb[0], M[0], (int)rows[1], (int)G[1], M[1])
+  if (xv <= 1) OKQ_MIXED(1);
+  else if (xv == 2) OKQ_MIXED(2);
+  else OKQ_MIXED(4);
+#undef OKQ_MIXED
+  return hipGetLastError();
 }
 
 hipError_t launch_gemv(int type, const float *x, int64_t K, const void *w, int64_t N, const float *bias, float *y,

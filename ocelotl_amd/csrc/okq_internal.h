@@ -57,12 +57,22 @@ constexpr int kGemvMaxProblems = 4;
 // `a` and epsilon `eps`, or the gated SiLU silu(x) * a (x = gate, a = up).
 // A transform needs every matrix of the launch to pass gemv_streams.
 enum GemvProKind { kProNone = 0, kProRms = 1, kProSwiGLU = 2 };
+// `h` (two matrices that gemv_pairs accepts, gate then up, no bias, no
+// prologue): the launch also writes silu(gate) * up [N] there.
 struct GemvPro {
   int kind;
   const float *a;
   float eps;
+  float *h;
 };
 bool gemv_streams(int type, int64_t K, const void *w, int64_t N);
+bool gemv_pairs(int type, int64_t K, const void *gate, const void *up, int64_t N, int cu_count);
+// Q4_K and Q6_K matrices (at least one of each, types[i] per matrix) against
+// one activation row in one launch; each result is its own launch's bit for
+// bit.  gemv_mixes: every matrix streams.
+bool gemv_mixes(int64_t K, int count, const int *types, const void *const *w, const int64_t *N);
+hipError_t launch_gemv_mixed(const float *x, int64_t K, int count, const int *types, const void *const *w,
+                             const int64_t *N, const float *const *bias, float *const *y, int cu_count, hipStream_t s);
 // x [rows, K] and y[i] [rows, N[i]] row-major; every pass over the weights
 // serves up to four activation rows.  A prologue needs rows == 1.
 hipError_t launch_gemv_multi(int type, const float *x, int64_t K, int64_t rows, int count, const void *const *w,

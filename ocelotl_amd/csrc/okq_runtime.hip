@@ -756,6 +756,29 @@ okq_status okq_linear_multi_q(const float *x, int64_t rows, int64_t in_features,
       (pass == 0 ? n4 : n6) += 1;
     }
   }
+  if (rows == 1) {
+    // one row: the GEMV's Q4_K and Q6_K matrices in one launch
+    const void *mw[okq::kGemvMaxProblems];
+    int64_t mn[okq::kGemvMaxProblems];
+    const float *mb[okq::kGemvMaxProblems];
+    float *mo[okq::kGemvMaxProblems];
+    int types[okq::kGemvMaxProblems], c = 0;
+    for (int i = 0; i < count; ++i) {
+      if ((w_types[i] != OKQ_TYPE_Q4_K && w_types[i] != OKQ_TYPE_Q6_K) || out_features[i] <= 0) continue;
+      types[c] = (int)w_types[i];
+      mw[c] = w[i];
+      mn[c] = out_features[i];
+      mb[c] = b[i];
+      mo[c++] = out[i];
+    }
+    if (c > 1 && okq::gemv_mixes(in_features, c, types, mw, mn)) {
+      st = hip_status(okq::launch_gemv_mixed(x, in_features, c, types, mw, mn, mb, mo, info.cu_count, s),
+                      "linear_multi launch");
+      if (st != OKQ_OK) return st;
+      for (int i = 0; i < count; ++i)
+        taken[i] = (w_types[i] == OKQ_TYPE_Q4_K || w_types[i] == OKQ_TYPE_Q6_K) && out_features[i] > 0;
+    }
+  }
   if (rows > okq::kGemmDecodeRows) {
     // prefill: the matrices of every format that the MFMA kernels take share
     // one pre-pass and one reduction
@@ -869,7 +892,7 @@ okq_status okq_rmsnorm_linear_q_multi(const float *x, int64_t rows, int64_t hidd
   const float *nobias[okq::kGemvMaxProblems] = {nullptr, nullptr, nullptr, nullptr};
   const float *const *b = bias ? bias : nobias;
   if (rows == 1 && streams) {  // one decode row: every workgroup normalises x in its prologue
-    const okq::GemvPro pro{okq::kProRms, norm_weight, epsilon};
+    const okq::GemvPro pro{okq::kProRms, norm_weight, epsilon, nullptr};
     for (int64_t r = 0; r < rows; ++r) {
       float *o[okq::kGemvMaxProblems];
       for (int i = 0; i < count; ++i) o[i] = out[i] + r * out_features[i];
@@ -928,6 +951,26 @@ okq_status okq_mlp_gated_silu_q(const float *x, int64_t rows, int64_t hidden, in
   // GEMV pass over both weights, or one decode-batch launch, whose split-K
   // reduction then applies the SiLU too)
   bool swiglu_done = false;
+  // one row, a down weight that streams: gate and up row by row in pairs, so
+  // that their launch also leaves silu(gate) * up in the neighbours' workspace
+  // and the down GEMV reads it as it is (without that workspace -- a capture
+  // before any such call -- the prologue below computes it)
+  void *hbuf = nullptr;
+  if (rows == 1 && gate_type == up_type && okq::gemv_streams((int)down_type, intermediate, down_w, hidden) &&
+      okq::gemv_pairs((int)gate_type, hidden, gate_w, up_w, intermediate, info.cu_count) &&
+      get_workspace(dev, s, (size_t)intermediate * sizeof(float), &hbuf, 1) == OKQ_OK) {
+    const void *const gw[2] = {gate_w, up_w};
+    const int64_t ns[2] = {intermediate, intermediate}, nd = hidden;
+    const float *const nob[2] = {nullptr, nullptr};
+    float *const os[2] = {gate_buf, up_buf};
+    float *const h = static_cast<float *>(hbuf);
+    hipError_t e = okq::launch_gemv_multi((int)gate_type, x, hidden, 1, 2, gw, ns, nob, os, info.cu_count, s,
+                                          okq::GemvPro{okq::kProNone, nullptr, 0.0f, h});
+    if (e == hipSuccess)
+      e = okq::launch_gemv_multi((int)down_type, h, intermediate, 1, 1, &down_w, &nd, nob, &out, info.cu_count, s,
+                                 okq::GemvPro{});
+    return hip_status(e, "mlp launch");
+  }
   if (gate_type == up_type) {
     const void *ws[2] = {gate_w, up_w};
     const uint64_t wb[2] = {gate_bytes, up_bytes};
@@ -949,7 +992,7 @@ okq_status okq_mlp_gated_silu_q(const float *x, int64_t rows, int64_t hidden, in
   // gate_buf (the reference's final content of gate_buf) for the other paths:
   // by gate/up's split-K reduction, else by its own pass
   if (rows == 1 && okq::gemv_streams((int)down_type, intermediate, down_w, hidden)) {
-    const okq::GemvPro base{okq::kProSwiGLU, nullptr, 0.0f};
+    const okq::GemvPro base{okq::kProSwiGLU, nullptr, 0.0f, nullptr};
     const float *nob = nullptr;
     for (int64_t r = 0; r < rows; ++r) {
       okq::GemvPro pro = base;

@@ -115,3 +115,42 @@ def test_linear_multi_q_repeats_bit_for_bit(torch, okq, orc):
         runs.append([o.cpu().numpy() for o in outs])
     for a, b in zip(*runs):
         assert (a.view(np.uint32) == b.view(np.uint32)).all()
+
+
+@pytest.mark.parametrize("k,mats", [
+    (4096, [(O.Q4_K, 4096), (O.Q4_K, 1024), (O.Q6_K, 1024)]),   # q, k, v of a Llama-3-8B layer
+    (4096, [(O.Q6_K, 33), (O.Q4_K, 5), (O.Q6_K, 300), (O.Q4_K, 2)]),
+    (14336, [(O.Q6_K, 256), (O.Q4_K, 4096)]),                   # teams of four waves
+    (256, [(O.Q4_K, 20000), (O.Q6_K, 8)]),                      # many rows of one block beside a few
+    (1024, [(O.Q4_K, 64), (O.Q6_K, 31), (O.Q8_0, 128)]),        # Q8_0 stays on its own launch
+])
+@pytest.mark.parametrize("special", [None, "outlier", "inf"])
+def test_one_row_of_two_formats_shares_a_launch_bit_for_bit(torch, okq, orc, k, mats, special):
+    """One activation row through Q4_K and Q6_K matrices: one GEMV launch, each
+    output its own call's bit for bit, also with a wide run (three limbs) and
+    on the IEEE path."""
+    import ctypes
+    print(f"[gpu] mixed one row K={k} mats={mats} {special}", flush=True)
+    x = orc.normal(9900 + k, k, 1.0)
+    if special == "outlier":
+        x[k // 2] = 300.0
+    if special == "inf":
+        x[5], x[k - 1] = -np.inf, np.nan
+    xd = _dev(torch, x)
+    wds = [_dev(torch, orc.quantize(t, orc.normal(9910 + i, n * k, 0.02))) for i, (t, n) in enumerate(mats)]
+    bds = [_dev(torch, orc.normal(9920 + i, n, 0.1)) if i % 2 == 0 else None for i, (_, n) in enumerate(mats)]
+    outs = [torch.full((n,), 7.0, dtype=torch.float32, device="cuda") for _, n in mats]
+    arr = lambda ty, vals: (ty * len(mats))(*vals)
+    s = torch.cuda.current_stream().cuda_stream
+    okq.call("okq_linear_multi_q", xd.data_ptr(), 1, k, len(mats), arr(ctypes.c_uint32, [t for t, _ in mats]),
+             arr(ctypes.c_void_p, [w.data_ptr() for w in wds]), arr(ctypes.c_uint64, [w.numel() for w in wds]),
+             arr(ctypes.c_int64, [n for _, n in mats]),
+             arr(ctypes.c_void_p, [None if b is None else b.data_ptr() for b in bds]),
+             arr(ctypes.c_void_p, [o.data_ptr() for o in outs]), s)
+    for (t, n), w, b, o in zip(mats, wds, bds, outs):
+        one = torch.full((n,), 5.0, dtype=torch.float32, device="cuda")
+        okq.call("okq_linear_out_by_in_q", xd.data_ptr(), 1, k, t, w.data_ptr(), w.numel(), n,
+                 None if b is None else b.data_ptr(), one.data_ptr(), s)
+        torch.cuda.synchronize()
+        got, want = o.cpu().numpy(), one.cpu().numpy()
+        assert ((got.view(np.uint32) == want.view(np.uint32)) | (np.isnan(got) & np.isnan(want))).all(), (t, n)

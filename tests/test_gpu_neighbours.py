@@ -363,3 +363,64 @@ def test_mlp_gated_silu_q_validates_before_launch(torch, okq, orc):
     assert e.value.status == okq.E_SHAPE and "down projection" in e.value.message
     torch.cuda.synchronize()
     assert (out.cpu().numpy() == 7.0).all()
+
+
+@pytest.mark.parametrize("tgu,td,hidden,inter,special", [
+    (O.Q4_K, O.Q6_K, 4096, 14336, None),
+    (O.Q8_0, O.Q8_0, 1024, 8256, None),        # the least rows that go in pairs, plus a ragged step
+    (O.Q5_K, O.Q5_K, 2048, 8448, "outlier"),   # a wide run: three limbs
+    (O.Q4_K, O.Q4_K, 1024, 9216, "inf"),       # infinities and a NaN: the IEEE path
+])
+def test_mlp_one_row_in_pairs_matches_the_grouped_calls(torch, okq, orc, tgu, td, hidden, inter, special):
+    """One row whose gate and up rows go through the GEMV in pairs: gate_buf and
+    up_buf equal okq_gemv_multi's outputs bit for bit, and out equals, bit for
+    bit, the same call captured on a stream that holds no workspace yet, whose
+    down launch computes the SiLU itself."""
+    print(f"[gpu] mlp pairs types={tgu},{td} hidden={hidden} inter={inter} {special}", flush=True)
+    x = orc.normal(7600 + hidden, hidden, 1.0)
+    if special == "outlier":
+        x[17] = 300.0
+    if special == "inf":
+        x[3], x[40], x[41] = np.inf, np.nan, -np.inf
+    gd, ud, dd = (_dev(torch, orc.quantize(t, orc.normal(7601 + i, n * k, 0.02)))
+                  for i, (t, n, k) in enumerate([(tgu, inter, hidden), (tgu, inter, hidden), (td, hidden, inter)]))
+    xd = _dev(torch, x)
+
+    def mlp(stream):
+        gb, ub, out = (torch.full((n,), 7.0, device="cuda") for n in (inter, inter, hidden))
+        return gb, ub, out, lambda: okq.call(
+            "okq_mlp_gated_silu_q", xd.data_ptr(), 1, hidden, inter, tgu, gd.data_ptr(), gd.numel(), tgu,
+            ud.data_ptr(), ud.numel(), td, dd.data_ptr(), dd.numel(), gb.data_ptr(), ub.data_ptr(), out.data_ptr(),
+            stream)
+
+    gb, ub, out, call = mlp(_stream(torch))
+    call()
+    g2, u2 = torch.full((inter,), 7.0, device="cuda"), torch.full((inter,), 7.0, device="cuda")
+    okq.call("okq_gemv_multi", xd.data_ptr(), 1, hidden, tgu, 2, (ctypes.c_void_p * 2)(gd.data_ptr(), ud.data_ptr()),
+             (ctypes.c_uint64 * 2)(gd.numel(), ud.numel()), (ctypes.c_int64 * 2)(inter, inter), None,
+             (ctypes.c_void_p * 2)(g2.data_ptr(), u2.data_ptr()), _stream(torch))
+    torch.cuda.synchronize()
+    assert _same_bits(gb.cpu(), g2.cpu()).all() and _same_bits(ub.cpu(), u2.cpu()).all()
+    first = out.cpu().numpy().copy()
+    out.fill_(7.0)
+    call()
+    torch.cuda.synchronize()
+    assert _same_bits(out.cpu(), first).all()
+    # hipStreamNonBlocking streams of torch's pool may have served other
+    # tests, so the capture runs on a stream made for it
+    hip = ctypes.CDLL("libamdhip64.so")
+    raw = ctypes.c_void_p()
+    assert hip.hipStreamCreate(ctypes.byref(raw)) == 0
+    side = torch.cuda.ExternalStream(raw.value)
+    gb3, ub3, out3, call3 = mlp(raw.value)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        call3()
+    for _ in range(3):
+        out3.fill_(7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert _same_bits(gb3.cpu(), g2.cpu()).all() and _same_bits(ub3.cpu(), u2.cpu()).all()
+        assert _same_bits(out3.cpu(), first).all()
+    assert np.isnan(first).all() if special == "inf" else np.isfinite(first).all()
