@@ -17,20 +17,13 @@
 //     is one extra K=16 MFMA per super-block on (xsum hi, xsum lo) x m.
 //   So every product inside an MFMA is exact and only f32 summation rounds.
 //
-// Layout / schedule (gfx950):
+// This file holds what the prefill kernels share (above 32 rows:
+// okq_gemm_f32.hip, okq_gemm_wide.hip, okq_gemm_pair.hip, okq_gemm_q6.hip,
+// okq_gemm_q8.hip), the decode-batch kernel (up to 32 rows), the split-K
+// reductions and the plans.
 //   * A pre-pass (one workgroup per row) converts X once per call into a
 //     workspace: fp16 planes [M][K], per-32 sums [M][K/32] as fp16 (hi, lo)
 //     pairs (<= 32768 after scaling) and the row scales 2^s [M].
-//   * Workgroup tile 256 x 128 (8 waves) or 128 x 128 (4 waves) when 256-row
-//     tiles would leave CUs idle; each wave owns 64 x 64 = 2 x 2 MFMA 32x32x16
-//     tiles.  K advances in steps of one 64-weight Q4_K chunk through a
-//     software pipeline: raw loads two steps ahead in registers, the B
-//     dequantisation (GGUF blocks -> fp16 sc*q) of step i+1 overlapping the
-//     MFMAs of step i, double-buffered LDS, one barrier per step.
-//   * Tiles are ordered so consecutive tiles (the M-tiles of one N-tile) land
-//     on one XCD: workgroup b runs on XCD b % 8, so b is remapped to give each
-//     XCD a contiguous range of tiles and the weight tile is re-read from that
-//     XCD's L2.
 #include <algorithm>
 #include <type_traits>
 
@@ -53,8 +46,6 @@ __device__ __forceinline__ Rsrc make_rsrc(const void *base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), (short)0, (int)bytes, 0x00020000);
 }
 __device__ __forceinline__ u32x4 bload4(Rsrc r, uint32_t off) { return __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0); }
-
-constexpr int kBN = 128;
 
 // ---------------------------------------------------------------------------
 // pre-pass: X -> fp16 planes + per-32 sums, one workgroup per row
@@ -301,41 +292,6 @@ __device__ __forceinline__ void nib4(uint32_t n4, h2 sc2, h2 off2, h2 &p0, h2 &p
   p1 = nib_pair(__builtin_amdgcn_perm(0x64646464u, n4, 0x04030402u), sc2, off2);
 }
 
-// ---------------------------------------------------------------------------
-// main kernel
-// ---------------------------------------------------------------------------
-constexpr int kKB = 64;         // K per pipeline step: one 64-weight Q4_K chunk
-constexpr int kLDB = kKB + 8;   // LDS row pitch in halves (spreads rows over banks)
-
-template <int BM, bool kLo, int kFmt>
-struct alignas(16) GemmSmem {
-  static constexpr bool kMins = kFmt == kQ4_K || kFmt == kQ5_K;
-  _Float16 A[2][BM][kLDB];
-  _Float16 Alo[2][kLo ? BM : 1][kLDB];
-  _Float16 B[2][kBN][kLDB];
-  _Float16 Blo[2][kFmt == kQ6_K || kFmt == kQ8_0 ? kBN : 1][kLDB];  // Q6_K, Q8_0: the exact remainder plane
-  _Float16 xs[2][kMins ? BM : 1][16];   // per super-block parity: xsum hi/lo of sub-blocks 0..7
-  _Float16 mn[2][kMins ? kBN : 1][16];  // per super-block parity: 6-bit mins, each twice
-  float d[2][kBN], dmin[2][kMins ? kBN : 1];
-};
-
-// Raw global data of one pipeline step for one thread.
-template <int BM, bool kLo, int kFmt>
-struct StepRegs {
-  u32x4 a[4], al[kLo ? 4 : 1];  // 32 activations (fp16) of one row
-  u32x4 xs;                     // 4 (hi, lo) xsum pairs (first chunk of a super-block)
-  u32x4 hd;                     // Q4_K header of the weight row's super-block
-  u32x4 q;                      // 16 (BM=128) or 8 (BM=256, in .x/.y) qs bytes
-  u32x4 qh;                     // Q5_K: the qh bytes of the same l (fifth bits)
-  // Q6_K (BM = 128): dword windows (5 dwords for 16 bytes) of the ql bytes of
-  // k < 32, of k >= 32 and of the qh bytes; 3 dwords around the half's 8
-  // scales; d (2-byte load, first chunk of a super-block)
-  uint32_t l0[kFmt == kQ6_K ? 5 : 1], l1[kFmt == kQ6_K ? 5 : 1], hq[kFmt == kQ6_K ? 5 : 1];
-  uint32_t sc[kFmt == kQ6_K ? 3 : 1], dw;
-  // Q8_0 (BM = 128): the dword window of this thread's 34-byte block
-  uint32_t q8[kFmt == kQ8_0 ? 9 : 1];
-};
-
 // v = sc * (q - 32) for the four 6-bit values in the bytes of q4, as two
 // exact fp16 planes v = hi + lo: 0x64|q is the fp16 1024 + q, minus 1056
 // gives q - 32 exactly; hi = fp16(v) is exact while |v| <= 2048 and rounds to
@@ -369,432 +325,6 @@ __device__ __forceinline__ void q8_4(uint32_t q4, h2 d2, h2 &p0, h2 &p1, h2 &l0,
   l1 = __builtin_elementwise_fma(c, d2, -p1);
 }
 
-// BM x 128 workgroup tile, BM/32 waves arranged (BM/64) x 2, each 64 x 64.
-// Software pipeline over 64-wide K steps: raw loads run two steps ahead in
-// registers, the dequantisation of step i+1 overlaps the MFMAs of step i, LDS
-// is double buffered, one barrier per step.
-template <int BM, bool kLo, int kFmt>
-__global__ __launch_bounds__(BM * 2) void gemm_kq_kernel(const _Float16 *__restrict__ xhi,
-                                                         const _Float16 *__restrict__ xlo,
-                                                         const h2 *__restrict__ xsum, const float *__restrict__ rscale,
-                                                         const uint8_t *__restrict__ W, const float *__restrict__ bias,
-                                                         float *__restrict__ Y, int M, int N, int K, int tiles_m,
-                                                         int tiles, int ksplit, float *__restrict__ part) {
-  constexpr int NT = BM * 2;       // threads
-  constexpr int TPR = NT / kBN;    // B-staging threads per weight row (2 or 4)
-  constexpr int QB = 32 / TPR;     // qs bytes per thread per step (16 or 8)
-  constexpr bool kQ6 = kFmt == kQ6_K, kQ8 = kFmt == kQ8_0, kQ5 = kFmt == kQ5_K;
-  static_assert(!kQ6 || QB == 16, "Q6_K staging takes 16-byte windows (BM = 128)");
-  static_assert(!kQ8 || TPR == 2, "Q8_0 staging takes one 34-byte block per thread (BM = 128)");
-  // bytes per 256 weights of a row: one super-block, or eight Q8_0 blocks
-  constexpr uint32_t kBlk = kQ6 ? kQ6KBytes : kQ8 ? 8 * kQ8Bytes : kQ5 ? kQ5KBytes : kQ4KBytes;
-  __shared__ GemmSmem<BM, kLo, kFmt> sm;
-  // XCD-aware tile order: workgroup b runs on XCD b % 8; give each XCD a
-  // contiguous range of tiles (consecutive tiles share an N-tile).
-  // With split-K (ksplit > 1) workgroup (tile, z) covers super-blocks
-  // [z * nsb_all / ksplit, (z + 1) * nsb_all / ksplit) and writes its f32
-  // partial tile to part[z]; consecutive indices keep one slice z and walk
-  // the M-tiles of an N-tile (they share the weight tile in L2).
-  const int b = (int)blockIdx.x;
-  const int jobs = tiles * ksplit;
-  const int per_xcd = (jobs + 7) / 8;
-  const int job = (b % 8) * per_xcd + b / 8;
-  if (job >= jobs) return;
-  const int z = job / tiles, tile = job % tiles;
-  const int m0 = (tile % tiles_m) * BM;
-  const int n0 = (tile / tiles_m) * kBN;
-
-  const int tid = (int)threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int nsb_all = K / 256;
-  const int sb0 = (int)((int64_t)z * nsb_all / ksplit);
-  const int nsb = (int)((int64_t)(z + 1) * nsb_all / ksplit) - sb0;  // super-blocks of this slice
-  const uint32_t row_bytes = (uint32_t)nsb_all * kBlk;
-
-  const int sr = tid >> 1, sp = tid & 1;        // A: row, 32-wide half
-  const int br = tid / TPR, bq = tid % TPR;     // B: weight row, byte window
-  const uint32_t K32 = (uint32_t)K;
-  const Rsrc rs_xh = make_rsrc(xhi, (uint32_t)((size_t)M * K * 2));
-  const Rsrc rs_xl = make_rsrc(kLo ? xlo : xhi, (uint32_t)((size_t)M * K * 2));
-  const Rsrc rs_xs = make_rsrc(xsum, (uint32_t)((size_t)M * (K / 32) * 4));
-  const Rsrc rs_w = make_rsrc(W, (uint32_t)((size_t)N * row_bytes));
-  // byte offsets of this thread's rows (past the end for rows >= M / >= N:
-  // the descriptors return zeros there)
-  const uint32_t a_row = (uint32_t)(m0 + sr) * K32 * 2u + 64u * (uint32_t)sp + 512u * (uint32_t)sb0;
-  const uint32_t s_row = (uint32_t)(m0 + sr) * (K32 / 32u) * 4u + 16u * (uint32_t)sp + 32u * (uint32_t)sb0;
-  const uint32_t w_row = (uint32_t)(n0 + br) * row_bytes + (uint32_t)sb0 * kBlk;
-
-  // C = step & 3 is a compile-time constant at every call site, so the body
-  // is straight-line code (no divergent branches around the loads: the wait
-  // counters then only wait for the step actually consumed).  Steps past the
-  // end read inside the next row or past the descriptor (zeros); unused.
-  auto load = [&](StepRegs<BM, kLo, kFmt> &r, int step, auto Cc) {
-    constexpr int c = decltype(Cc)::value;
-    const int sb = step >> 2;
-    const uint32_t ka = a_row + 2u * (uint32_t)(step * kKB);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) r.a[i] = bload4(rs_xh, ka + 16u * i);
-    if (kLo) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) r.al[i] = bload4(rs_xl, ka + 16u * i);
-    }
-    if constexpr (kQ8) {
-      // blocks 2c and 2c + 1 of the super-block hold this step's 64 weights;
-      // thread bq stages block 2c + bq: a 9-dword window from the dword below
-      // its (2-byte aligned) start
-      const uint32_t B = w_row + (uint32_t)sb * kBlk + (2u * c + (uint32_t)bq) * kQ8Bytes;
-      const uint32_t a = B & ~3u;
-      const u32x4 v0 = bload4(rs_w, a), v1 = bload4(rs_w, a + 16u);
-      r.q8[0] = v0.x, r.q8[1] = v0.y, r.q8[2] = v0.z, r.q8[3] = v0.w;
-      r.q8[4] = v1.x, r.q8[5] = v1.y, r.q8[6] = v1.z, r.q8[7] = v1.w;
-      r.q8[8] = __builtin_amdgcn_raw_buffer_load_b32(rs_w, a + 32u, 0, 0);
-      return;
-    }
-    if constexpr (kQ6) {
-      // chunk c of the super-block: half h = c / 2 (ql bytes 64h.., qh bytes
-      // 128 + 32h..); this thread's l = 16 bq .. 16 bq + 15.  Windows start at
-      // the dword below each (2-byte aligned) field.
-      constexpr uint32_t h = c >> 1;
-      const uint32_t B = w_row + (uint32_t)sb * kBlk;
-      auto win = [&](uint32_t *dst, uint32_t at, int n) {
-#pragma unroll
-        for (int t = 0; t < n; ++t) dst[t] = __builtin_amdgcn_raw_buffer_load_b32(rs_w, (at & ~3u) + 4u * t, 0, 0);
-      };
-      // both chunks of a half use the same bytes (the second read hits the cache)
-      win(r.l0, B + 64u * h + 16u * bq, 5);
-      win(r.l1, B + 64u * h + 32u + 16u * bq, 5);
-      win(r.hq, B + 128u + 32u * h + 16u * bq, 5);
-      win(r.sc, B + 192u + 8u * h, 3);
-      // d with a 2-byte load: a dword window could end past the tensor (whose
-      // size is only 2-byte aligned) and the range check would zero it
-      if constexpr (c == 0) r.dw = (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(rs_w, B + 208u, 0, 0);
-      return;
-    }
-    if constexpr (c == 0) r.xs = bload4(rs_xs, s_row + 32u * (uint32_t)sb);
-    // Q4_K / Q5_K: the header, this thread's QB qs bytes of chunk c and
-    // (Q5_K) the qh bytes of the same positions l
-    const uint32_t blk = w_row + (uint32_t)sb * kBlk;
-    r.hd = bload4(rs_w, blk);
-    const uint32_t qo = blk + (kQ5 ? 48u : 16u) + 32u * (uint32_t)c + (uint32_t)(QB * bq);
-    if (QB == 16) {
-      r.q = bload4(rs_w, qo);
-      if (kQ5) r.qh = bload4(rs_w, blk + 16u + (uint32_t)(QB * bq));
-    } else {
-      const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(rs_w, qo, 0, 0);
-      r.q = u32x4{v.x, v.y, 0u, 0u};
-      if (kQ5) {
-        const u32x2 h = __builtin_amdgcn_raw_buffer_load_b64(rs_w, blk + 16u + (uint32_t)(QB * bq), 0, 0);
-        r.qh = u32x4{h.x, h.y, 0u, 0u};
-      }
-    }
-  };
-
-  auto stage = [&](const StepRegs<BM, kLo, kFmt> &r, int step, int buf, auto Cc) {
-    constexpr int c = decltype(Cc)::value;
-    const int sbp = (step >> 2) & 1;
-    u32x4 *da = reinterpret_cast<u32x4 *>(&sm.A[buf][sr][32 * sp]);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) da[i] = r.a[i];
-    if (kLo) {
-      u32x4 *dl = reinterpret_cast<u32x4 *>(&sm.Alo[buf][sr][32 * sp]);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) dl[i] = r.al[i];
-    }
-    if constexpr (kQ8) {
-      const uint32_t B = w_row + (uint32_t)(step >> 2) * kBlk + (2u * c + (uint32_t)bq) * kQ8Bytes;
-      const uint32_t ra = B & 3u;
-      uint32_t wv[9];  // bytes B + 4i .. of the block (realigned window)
-#pragma unroll
-      for (int t = 0; t < 8; ++t) wv[t] = __builtin_amdgcn_alignbyte(r.q8[t + 1], r.q8[t], ra);
-      wv[8] = __builtin_amdgcn_alignbyte(0u, r.q8[8], ra);
-      const _Float16 dh = __builtin_bit_cast(_Float16, (uint16_t)(wv[0] & 0xffffu));
-      const h2 d2 = {dh, dh};
-      h2 hi[16], lo[16];
-#pragma unroll
-      for (int w = 0; w < 8; ++w) {
-        const uint32_t q4 = __builtin_amdgcn_alignbyte(wv[w + 1], wv[w], 2u);  // quants 4w .. 4w + 3
-        q8_4(q4, d2, hi[2 * w], hi[2 * w + 1], lo[2 * w], lo[2 * w + 1]);
-      }
-      auto put = [&](_Float16 *dst, const h2 *v) {
-        u32x4 *d4 = reinterpret_cast<u32x4 *>(dst);
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-          d4[t] = u32x4{__builtin_bit_cast(uint32_t, v[4 * t]), __builtin_bit_cast(uint32_t, v[4 * t + 1]),
-                        __builtin_bit_cast(uint32_t, v[4 * t + 2]), __builtin_bit_cast(uint32_t, v[4 * t + 3])};
-      };
-      put(&sm.B[buf][br][32 * bq], hi);
-      put(&sm.Blo[buf][br][32 * bq], lo);
-      return;
-    }
-    if constexpr (kQ6) {
-      constexpr uint32_t cc = c & 1, h = c >> 1;
-      const uint32_t B = w_row + (uint32_t)(step >> 2) * kBlk;
-      // realign each window by the field's offset within its first dword
-      auto bytes16 = [&](const uint32_t *w, uint32_t at, uint32_t o[4]) {
-        const uint32_t ra = at & 3u;
-#pragma unroll
-        for (int t = 0; t < 4; ++t) o[t] = __builtin_amdgcn_alignbyte(w[t + 1], w[t], ra);
-      };
-      uint32_t L0[4], L1[4], H[4];
-      bytes16(r.l0, B + 64u * h + 16u * bq, L0);
-      bytes16(r.l1, B + 64u * h + 32u + 16u * bq, L1);
-      bytes16(r.hq, B + 128u + 32u * h + 16u * bq, H);
-      // int8 scales of this thread's l-run (l / 16 = bq): index 8h + bq + 2p
-      // for p = 2cc (k < 32) and 2cc + 1 (k >= 32)
-      const uint32_t sat = B + 192u + 8u * h;
-      const uint32_t s0 = __builtin_amdgcn_alignbyte(r.sc[1], r.sc[0], sat & 3u);
-      const uint32_t s1 = __builtin_amdgcn_alignbyte(r.sc[2], r.sc[1], sat & 3u);
-      const uint32_t ia = (uint32_t)bq + 4u * cc, ib = ia + 2u;  // 0..7
-      const int sca = (int)__builtin_amdgcn_sbfe((int)(ia < 4 ? s0 : s1), 8 * (ia & 3u), 8u);
-      const int scb = (int)__builtin_amdgcn_sbfe((int)(ib < 4 ? s0 : s1), 8 * (ib & 3u), 8u);
-      const _Float16 fa = (_Float16)(float)sca, fb = (_Float16)(float)scb;
-      const h2 sa = {fa, fa}, sbv = {fb, fb};
-      // first: k < 32 of the chunk, second: k >= 32; r*: the remainder plane
-      h2 fi[8], se[8], rf[8], rs[8];
-#pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        const uint32_t qa = ((L0[w] >> (4 * cc)) & 0x0F0F0F0Fu) | (((H[w] >> (4 * cc)) & 0x03030303u) << 4);
-        const uint32_t qb = ((L1[w] >> (4 * cc)) & 0x0F0F0F0Fu) | (((H[w] >> (4 * cc + 2)) & 0x03030303u) << 4);
-        q6_4(qa, sa, fi[2 * w], fi[2 * w + 1], rf[2 * w], rf[2 * w + 1]);
-        q6_4(qb, sbv, se[2 * w], se[2 * w + 1], rs[2 * w], rs[2 * w + 1]);
-      }
-      auto put = [&](_Float16 *dst, const h2 *v) {
-        u32x4 *d4 = reinterpret_cast<u32x4 *>(dst);
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-          d4[t] = u32x4{__builtin_bit_cast(uint32_t, v[4 * t]), __builtin_bit_cast(uint32_t, v[4 * t + 1]),
-                        __builtin_bit_cast(uint32_t, v[4 * t + 2]), __builtin_bit_cast(uint32_t, v[4 * t + 3])};
-      };
-      put(&sm.B[buf][br][16 * bq], fi);
-      put(&sm.B[buf][br][32 + 16 * bq], se);
-      put(&sm.Blo[buf][br][16 * bq], rf);
-      put(&sm.Blo[buf][br][32 + 16 * bq], rs);
-      if constexpr (c == 0) sm.d[sbp][br] = f16_bits_hw(r.dw & 0xffffu);
-      return;
-    }
-    if constexpr (c == 0) *reinterpret_cast<u32x4 *>(&sm.xs[sbp][sr][8 * sp]) = r.xs;
-    // low nibbles -> sub-block 2c (k = byte), high nibbles -> 2c+1 (k = 32 + byte)
-    uint32_t sc0, mv0, sc1, mv1;
-    q4k_scale_min(2 * c, r.hd.y, r.hd.z, r.hd.w, sc0, mv0);
-    q4k_scale_min(2 * c + 1, r.hd.y, r.hd.z, r.hd.w, sc1, mv1);
-    const _Float16 s0 = (_Float16)(float)sc0, s1 = (_Float16)(float)sc1;
-    const _Float16 o0 = (_Float16)(-1024.0f * (float)sc0), o1 = (_Float16)(-1024.0f * (float)sc1);
-    const h2 sc0v = {s0, s0}, sc1v = {s1, s1}, off0 = {o0, o0}, off1 = {o1, o1};
-    constexpr int NW = QB / 4;
-    const uint32_t q[4] = {r.q.x, r.q.y, r.q.z, r.q.w};
-    const uint32_t qh[4] = {r.qh.x, r.qh.y, r.qh.z, r.qh.w};
-    h2 lo[2 * NW], hi[2 * NW];
-#pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      // Q5_K: bit 2c of qh[l] is bit 4 of the low nibble's value, bit 2c + 1
-      // of the high one's (sc * q <= 63 * 31 stays an exact fp16 integer)
-      const uint32_t f0 = kQ5 ? ((qh[w] >> (2 * c)) & 0x01010101u) << 4 : 0u;
-      const uint32_t f1 = kQ5 ? ((qh[w] >> (2 * c + 1)) & 0x01010101u) << 4 : 0u;
-      nib4((q[w] & 0x0F0F0F0Fu) | f0, sc0v, off0, lo[2 * w], lo[2 * w + 1]);
-      nib4(((q[w] >> 4) & 0x0F0F0F0Fu) | f1, sc1v, off1, hi[2 * w], hi[2 * w + 1]);
-    }
-    u32x4 *dlo = reinterpret_cast<u32x4 *>(&sm.B[buf][br][QB * bq]);
-    u32x4 *dhi = reinterpret_cast<u32x4 *>(&sm.B[buf][br][32 + QB * bq]);
-#pragma unroll
-    for (int i = 0; i < NW / 2; ++i) {
-      dlo[i] = u32x4{__builtin_bit_cast(uint32_t, lo[4 * i]), __builtin_bit_cast(uint32_t, lo[4 * i + 1]),
-                     __builtin_bit_cast(uint32_t, lo[4 * i + 2]), __builtin_bit_cast(uint32_t, lo[4 * i + 3])};
-      dhi[i] = u32x4{__builtin_bit_cast(uint32_t, hi[4 * i]), __builtin_bit_cast(uint32_t, hi[4 * i + 1]),
-                     __builtin_bit_cast(uint32_t, hi[4 * i + 2]), __builtin_bit_cast(uint32_t, hi[4 * i + 3])};
-    }
-    if constexpr (c == 0) {
-      // every staging thread of the row loaded the same header: all of them
-      // store the same values (no branch, so no conservative wait counters)
-      sm.d[sbp][br] = f16_bits_hw(r.hd.x & 0xffffu);
-      sm.dmin[sbp][br] = f16_bits_hw(r.hd.x >> 16);
-      h8 m0v, m1v;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        uint32_t scj, mj;
-        q4k_scale_min((uint32_t)j, r.hd.y, r.hd.z, r.hd.w, scj, mj);
-        const _Float16 mh = (_Float16)(float)mj;
-        if (j < 4) {
-          m0v[2 * j] = mh;
-          m0v[2 * j + 1] = mh;
-        } else {
-          m1v[2 * (j - 4)] = mh;
-          m1v[2 * (j - 4) + 1] = mh;
-        }
-      }
-      *reinterpret_cast<h8 *>(&sm.mn[sbp][br][0]) = m0v;
-      *reinterpret_cast<h8 *>(&sm.mn[sbp][br][8]) = m1v;
-    }
-  };
-
-  f16x acc[2][2], accs[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
-
-  // MFMA slice ks, lane group g = lane/32 covers k = 32g + 8ks + [0, 8) of the
-  // 64-wide step (the same k order as the direct-A kernel, so both kernels
-  // give bit-identical results for a row)
-  const int fr = lane & 31, fk = 8 * (lane >> 5), fk4 = 32 * (lane >> 5);
-  const f16x zero = {};
-
-  auto mma = [&](int buf, bool first) {
-#pragma unroll
-    for (int ks = 0; ks < kKB / 16; ++ks) {
-      h8 a[2], bv[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-        a[i] = *reinterpret_cast<const h8 *>(&sm.A[buf][wm * 64 + 32 * i + fr][fk4 + 8 * ks]);
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-        bv[j] = *reinterpret_cast<const h8 *>(&sm.B[buf][wn * 64 + 32 * j + fr][fk4 + 8 * ks]);
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          accs[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i], bv[j], (first && ks == 0) ? zero : accs[i][j],
-                                                              0, 0, 0);
-      if constexpr (kQ6 || kQ8) {  // the exact remainder plane of the weights (x_lo * remainder is below 2^-22)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const h8 bl = *reinterpret_cast<const h8 *>(&sm.Blo[buf][wn * 64 + 32 * j + fr][fk4 + 8 * ks]);
-#pragma unroll
-          for (int i = 0; i < 2; ++i)
-            accs[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i], bl, accs[i][j], 0, 0, 0);
-        }
-      }
-      if (kLo) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-          a[i] = *reinterpret_cast<const h8 *>(&sm.Alo[buf][wm * 64 + 32 * i + fr][fk4 + 8 * ks]);
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j)
-            accs[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i], bv[j], accs[i][j], 0, 0, 0);
-      }
-    }
-  };
-
-  // end of a super-block: acc += d * accs - dmin * (xsum . m)  (Q6_K: d * accs)
-  auto scale = [&](int sbp) {
-    if constexpr (kQ8) {  // d is inside the B planes
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-          for (int e = 0; e < 16; ++e) acc[i][j][e] += accs[i][j][e];
-      return;
-    }
-    if constexpr (kQ6) {
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const float dv = sm.d[sbp][wn * 64 + 32 * j + fr];
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int e = 0; e < 16; ++e) acc[i][j][e] = fmaf(dv, accs[i][j][e], acc[i][j][e]);
-      }
-      return;
-    }
-    h8 xa[2], mb[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) xa[i] = *reinterpret_cast<const h8 *>(&sm.xs[sbp][wm * 64 + 32 * i + fr][fk]);
-#pragma unroll
-    for (int j = 0; j < 2; ++j) mb[j] = *reinterpret_cast<const h8 *>(&sm.mn[sbp][wn * 64 + 32 * j + fr][fk]);
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int nn = wn * 64 + 32 * j + fr;
-      const float dv = sm.d[sbp][nn], dm = -sm.dmin[sbp][nn];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const f16x mins = __builtin_amdgcn_mfma_f32_32x32x16_f16(xa[i], mb[j], zero, 0, 0, 0);
-#pragma unroll
-        for (int e = 0; e < 16; ++e) acc[i][j][e] = fmaf(dm, mins[e], fmaf(dv, accs[i][j][e], acc[i][j][e]));
-      }
-    }
-  };
-
-  // Pipeline over steps i = 4*sb + c: LDS buffer i&1 holds step i while the
-  // register set of step i+1 is staged into the other buffer and step i+2 is
-  // in flight.
-  using C0 = std::integral_constant<int, 0>;
-  using C1 = std::integral_constant<int, 1>;
-  using C2 = std::integral_constant<int, 2>;
-  using C3 = std::integral_constant<int, 3>;
-  StepRegs<BM, kLo, kFmt> R0, R1;
-  load(R0, 0, C0{});
-  load(R1, 1, C1{});
-  stage(R0, 0, 0, C0{});
-  __syncthreads();
-  for (int sb = 0; sb < nsb; ++sb) {
-    const int i = 4 * sb;
-    load(R0, i + 2, C2{});
-    mma(0, true);
-    stage(R1, i + 1, 1, C1{});
-    __syncthreads();
-    load(R1, i + 3, C3{});
-    mma(1, false);
-    stage(R0, i + 2, 0, C2{});
-    __syncthreads();
-    load(R0, i + 4, C0{});
-    mma(0, false);
-    stage(R1, i + 3, 1, C3{});
-    __syncthreads();
-    load(R1, i + 5, C1{});
-    mma(1, false);
-    scale(sb & 1);
-    stage(R0, i + 4, 0, C0{});
-    __syncthreads();
-  }
-
-  // epilogue: C layout row = 8*(e/4) + 4*(lane/32) + e%4, col = lane%32
-  if (ksplit > 1) {  // raw partial tile; splitk_reduce_kernel scales and adds the bias
-    float *P = part + (size_t)z * M * N;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int col = n0 + wn * 64 + 32 * j + fr;
-      if (col >= N) continue;
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int row = m0 + wm * 64 + 32 * i + 8 * (e / 4) + 4 * (lane >> 5) + (e % 4);
-          if (row < M) P[(size_t)row * N + col] = acc[i][j][e];
-        }
-    }
-    return;
-  }
-  // undo the pre-pass's per-row power-of-two scale (exact)
-  float rs[2][16];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int row = m0 + wm * 64 + 32 * i + 8 * (e / 4) + 4 * (lane >> 5) + (e % 4);
-      rs[i][e] = row < M ? rscale[row] : 0.0f;
-    }
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int col = n0 + wn * 64 + 32 * j + fr;
-    if (col >= N) continue;
-    const float bv = bias ? bias[col] : 0.0f;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int row = m0 + wm * 64 + 32 * i + 8 * (e / 4) + 4 * (lane >> 5) + (e % 4);
-        // a NaN scale: the pre-pass wrote this row's IEEE outputs
-        if (row < M && !__builtin_isnan(rs[i][e])) Y[(size_t)row * N + col] = acc[i][j][e] * rs[i][e] + bv;
-      }
-    }
-  }
-}
-
 // ---------------------------------------------------------------------------
 // decode batches (2 <= M <= 16): a streaming kernel with MFMA contraction
 // ---------------------------------------------------------------------------
@@ -804,7 +334,7 @@ __global__ __launch_bounds__(BM * 2) void gemm_kq_kernel(const _Float16 *__restr
 // like the GEMV: a workgroup stages its K-slice of the activations (the
 // pre-pass planes) in LDS once, then every wave streams a sequence of items
 // (16-column tile, super-block) through a ring of D register sets with no
-// further barrier.  Operands and scaling are those of gemm_kq_kernel (exact
+// further barrier.  Operands and scaling are those of the prefill kernels (exact
 // fp16 products, per-super-block f32 scaling by d and dmin).
 //
 // MFMA v_mfma_f32_16x16x32_f16: lane l holds A[l % 16][8 (l / 16) + 0..7],
@@ -1125,7 +655,7 @@ struct DecQ6KT {
         const h8 ah = *reinterpret_cast<const h8 *>(ar[q] + ka);
         accs[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bh, accs[q], 0, 0, 0);
         accs[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bl, accs[q], 0, 0, 0);
-        if (kLo) {  // the x_lo * remainder term (below 2^-22 of the result) is left out, as in the tiled kernel
+        if (kLo) {  // the x_lo * remainder term (below 2^-22 of the result) is left out, as in okq_gemm_f32.hip
           const h8 al = *reinterpret_cast<const h8 *>(arl[q] + ka);
           accs[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bh, accs[q], 0, 0, 0);
         }
@@ -1221,7 +751,7 @@ struct DecQ80 {
 // The activations arrive raw (f32 when kLo, else bf16): every workgroup
 // converts its own K slice, so no pre-pass launch precedes the kernel.  Each
 // row of the slice is scaled by 2^-s so its largest |x| lies in [512, 1024)
-// (rows of zeros, infinities or NaNs keep s = 0), as the tiled kernel's
+// (rows of zeros, infinities or NaNs keep s = 0), as the prefill kernels'
 // pre-pass scales whole rows; the slice's outputs are multiplied back by 2^s
 // (exact), so split-K partials leave the kernel unscaled and
 // splitk_reduce_kernel only sums them in slice order and adds the bias.
@@ -1697,7 +1227,7 @@ __global__ __launch_bounds__(kDecWaves * 64) void gemm_decode_kernel(const void 
 }
 
 // Sum of the split-K partials in slice order (deterministic), then the row
-// scale (tiled kernel; the decode-batch kernel's partials are unscaled:
+// scale (the pre-pass's; Q8_0 bf16 partials have none:
 // rscale == nullptr) and the bias: Y[m, n] = (sum_z P[z][m, n]) * rscale[m] + bias[n].
 // Grid: 256-column blocks x rows (a row stride of gridDim.y beyond 65535
 // rows), so no thread divides its index.  The partials are read through a
@@ -1955,19 +1485,20 @@ bool gemm_supported(int type, int64_t M, int64_t K, int64_t N) {
   // 32-bit buffer offsets: activations (with a tile of padding rows) and weights
   const int64_t a_bytes = (M + 256) * K * 2;
   const int64_t sb_bytes = sb_bytes_of(type);
-  const int64_t w_bytes = (N + kBN) * (K / 256) * sb_bytes + 1024;
+  const int64_t w_bytes = (N + 128) * (K / 256) * sb_bytes + 1024;
   return (type == kQ4_K || type == kQ5_K || type == kQ6_K || type == kQ8_0) && K % 256 == 0 && N >= 1 && M >= 1 &&
          a_bytes < (int64_t)UINT32_MAX && w_bytes < (int64_t)UINT32_MAX;
 }
 
 static size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
 
-// K slices of gemm_f32_*_kernel for one matrix: the split of least estimated
-// time.  A round of workgroups (one per CU) takes ~7 us (Q4_K) per
-// super-block of its slice and ~5 us around its loop; the partials are
-// written and read once at ~4 TB/s, and their reduction is one more launch.
-static int64_t f32_split(int type, int64_t M, int64_t N, int64_t K, int cu_count) {
-  const double us_sb = (type == kQ6_K ? 10.0 : type == kQ8_0 ? 8.5 : 7.0) *
+// K slices of gemm_f32_kernel for one matrix: the split of least estimated
+// time.  A round of workgroups (one per CU) takes ~7 us (Q4_K, both planes;
+// one plane: the MFMAs of one) per super-block of its slice and ~5 us around
+// its loop; the partials are written and read once at ~4 TB/s, and their
+// reduction is one more launch.
+static int64_t f32_split(int type, int64_t M, int64_t N, int64_t K, bool one_plane, int cu_count) {
+  const double us_sb = (type == kQ6_K ? 10.0 : type == kQ8_0 ? 8.5 : 7.0) * (one_plane ? 0.7 : 1.0) *
                        (0.2 + 0.2 * gemm_f32_blocks(M));
   const int64_t nsb = K / 256, tiles = gemm_f32_tiles(M, N), cus = cu_count;
   int64_t best = 1;
@@ -1987,13 +1518,10 @@ static int64_t f32_split(int type, int64_t M, int64_t N, int64_t K, int cu_count
 GemmPlan gemm_plan(int type, int64_t M, int64_t N, int64_t K, bool x_is_bf16, int cu_count) {
   GemmPlan p{};
   p.kwaves = 1;
-  // More than 32 rows: Q4_K, Q5_K and Q8_0 with bf16 activations take the
-  // register-dequant kernels (okq_gemm_wide.hip, okq_gemm_pair.hip,
-  // okq_gemm_q8.hip); the tiled kernel takes the rest with 128 x 128 tiles
-  // (f32 activations need the second fp16 plane, which only fits the LDS
-  // budget at 128 rows; Q6_K stages its larger raw windows in the 4-wave
-  // tile's register budget), or 256 x 128 tiles for bf16 Q4_K shapes beyond
-  // the wide kernel's 32-bit offsets.
+  // More than 32 rows, weights dequantised in registers throughout: f32
+  // activations take okq_gemm_f32.hip; bf16 ones okq_gemm_wide.hip or
+  // okq_gemm_pair.hip (Q4_K, Q5_K), okq_gemm_q8.hip (Q8_0), okq_gemm_q6.hip
+  // (Q6_K grids that fill its tiles), okq_gemm_f32.hip with one plane otherwise.
   const int64_t nsb = K / 256;
   int64_t ks = 1;
   if (M <= kDecRows) {
@@ -2046,14 +1574,13 @@ GemmPlan gemm_plan(int type, int64_t M, int64_t N, int64_t K, bool x_is_bf16, in
     if (ks == 1 && mytiles > kDecMaxTiles)
       p.groups = (int)((ntiles + (int64_t)kDecWaves * kDecMaxTiles - 1) / ((int64_t)kDecWaves * kDecMaxTiles));
   } else {
-    // Q4_K, Q5_K and Q8_0 with bf16 activations: a kernel that dequantises
-    // the weights in registers; everything else: the tiled kernel.  Split K
-    // when the tiles alone leave CUs idle: enough slices for about one
-    // workgroup per CU, at least two super-blocks per slice, at most 8.
+    // Split K when the tiles alone leave CUs idle: enough slices for about one
+    // workgroup per CU, at least two super-blocks per slice, at most 8 (f32 and
+    // one-plane plans: f32_split).
     const bool reg_dequant = x_is_bf16 && gemm_wide_supported(type, M, K, N);
     // Q6_K with bf16 activations: gemm_wide_q6k_kernel (128 x 256 tiles, one
     // 8-wave workgroup per CU) while its (tile, K-slice) jobs fill at least
-    // 3/4 of their rounds of CUs; otherwise the tiled kernel
+    // 3/4 of their rounds of CUs; otherwise gemm_f32_kernel's smaller tiles
     bool q6_wide = false;
     int64_t q6_ks = 1;
     if (x_is_bf16 && type == kQ6_K) {
@@ -2065,7 +1592,7 @@ GemmPlan gemm_plan(int type, int64_t M, int64_t N, int64_t K, bool x_is_bf16, in
     if (!x_is_bf16) {
       p.bm = 128;
       p.wide = 5;
-      ks = f32_split(type, M, N, K, cu_count);
+      ks = f32_split(type, M, N, K, false, cu_count);
     } else if (type == kQ8_0) {
       // gemm_q8_kernel (bf16 activations straight from x: no pre-pass).  The
       // 8-wave 128 x 256 tiles (one workgroup per CU) while they fill at
@@ -2089,30 +1616,32 @@ GemmPlan gemm_plan(int type, int64_t M, int64_t N, int64_t K, bool x_is_bf16, in
       p.bm = 128;
       p.wide = 4;
       ks = q6_ks;
+    } else if (!reg_dequant) {
+      p.bm = 128;
+      p.wide = 6;
+      ks = f32_split(type, M, N, K, true, cu_count);
     } else {
-      p.bm = reg_dequant ? 128 : ((type == kQ4_K || type == kQ5_K) && x_is_bf16 && M > 128) ? 256 : 128;
+      p.bm = 128;
       const int64_t cus = cu_count;
-      const int64_t tiles = reg_dequant ? gemm_wide_tiles(M, N) : ((M + p.bm - 1) / p.bm) * ((N + kBN - 1) / kBN);
+      const int64_t tiles = gemm_wide_tiles(M, N);
       if (tiles * 4 < cus * 3) ks = std::min<int64_t>({(cus + tiles - 1) / tiles, nsb / 2, 8});
-      if (reg_dequant) {
-        // gemm_wide_q4k_kernel (128 x 256 tiles, one 8-wave workgroup per CU)
-        // while its workgroups fill at least 3/4 of their rounds of CUs (C4,
-        // us per call: M=512 gate 76.9 vs 86.7 for the other kernel, down 85.5
-        // vs 91.2, q 40.0 vs 41.1; M=2048 gate 292 vs 296, down 268 vs 301);
-        // otherwise gemm_pair_q4k_kernel (128 x 128 tiles, two 4-wave
-        // workgroups per CU), whose finer tiles and slices occupy every CU
-        // where the wide ones cannot (M=128 gate 39.5 vs 56.3, down 36.6 vs
-        // 42.8, q 24.2 vs 26.3; M=512 v 25.3 vs 27.8), with as many slices as
-        // fit one round of two workgroups per CU.
-        const int64_t jobs = tiles * std::max<int64_t>(1, ks);
-        const int64_t rounds = (jobs + cus - 1) / cus;
-        if (jobs * 4 >= rounds * cus * 3) {
-          p.wide = 1;
-        } else {
-          p.wide = 2;
-          const int64_t ptiles = gemm_pair_tiles(M, N), slots = 2 * cus;
-          ks = ptiles * 4 < slots * 3 ? std::max<int64_t>(1, std::min<int64_t>({slots / ptiles, nsb / 2, 8})) : 1;
-        }
+      // gemm_wide_q4k_kernel (128 x 256 tiles, one 8-wave workgroup per CU)
+      // while its workgroups fill at least 3/4 of their rounds of CUs (C4,
+      // us per call: M=512 gate 76.9 vs 86.7 for the other kernel, down 85.5
+      // vs 91.2, q 40.0 vs 41.1; M=2048 gate 292 vs 296, down 268 vs 301);
+      // otherwise gemm_pair_q4k_kernel (128 x 128 tiles, two 4-wave
+      // workgroups per CU), whose finer tiles and slices occupy every CU
+      // where the wide ones cannot (M=128 gate 39.5 vs 56.3, down 36.6 vs
+      // 42.8, q 24.2 vs 26.3; M=512 v 25.3 vs 27.8), with as many slices as
+      // fit one round of two workgroups per CU.
+      const int64_t jobs = tiles * std::max<int64_t>(1, ks);
+      const int64_t rounds = (jobs + cus - 1) / cus;
+      if (jobs * 4 >= rounds * cus * 3) {
+        p.wide = 1;
+      } else {
+        p.wide = 2;
+        const int64_t ptiles = gemm_pair_tiles(M, N), slots = 2 * cus;
+        ks = ptiles * 4 < slots * 3 ? std::max<int64_t>(1, std::min<int64_t>({slots / ptiles, nsb / 2, 8})) : 1;
       }
     }
   }
@@ -2305,35 +1834,6 @@ hipError_t launch_gemm_decode_mixed(const void *x, bool x_is_bf16, int64_t M, in
                        false);
 }
 
-// The tiled kernel over the pre-pass's plane (bf16 activations).
-static hipError_t launch_gemm_tiled(int type, _Float16 *xhi, h2 *xsum, float *rscale,
-                                    const uint8_t *W, const float *bias, float *y, int64_t M, int64_t N, int64_t K,
-                                    const GemmPlan &plan, float *part, hipStream_t s) {
-  const int m = (int)M, n = (int)N, k = (int)K, ks = plan.ksplit;
-  const int tiles_n = (int)((N + kBN - 1) / kBN);
-  const int tiles_m = (int)((M + plan.bm - 1) / plan.bm);
-  const int tiles = tiles_m * tiles_n;
-  const int per_xcd = (tiles * ks + 7) / 8;
-  const dim3 grid((unsigned)(per_xcd * 8)), block((unsigned)(plan.bm * 2));
-#define OKQ_GEMM(BM_, FMT_)                                                                                      \
-  launch_timed(gemm_kq_kernel<BM_, false, FMT_>, grid, block, 0u, s, xhi, nullptr, xsum, rscale, W, bias, y, m, n, k, \
-               tiles_m, tiles, ks, part)
-  if (type == kQ6_K) {
-    OKQ_GEMM(128, kQ6_K);
-  } else if (type == kQ8_0) {
-    OKQ_GEMM(128, kQ8_0);
-  } else if (type == kQ5_K) {
-    if (plan.bm == 256) OKQ_GEMM(256, kQ5_K);
-    else OKQ_GEMM(128, kQ5_K);
-  } else if (plan.bm == 256) {
-    OKQ_GEMM(256, kQ4_K);
-  } else {
-    OKQ_GEMM(128, kQ4_K);
-  }
-#undef OKQ_GEMM
-  return hipGetLastError();
-}
-
 static PrepIeee prep_ieee(int type, int64_t K, const void *w, int64_t N, const float *bias, float *y) {
   return PrepIeee{static_cast<const uint8_t *>(w), bias, y, (size_t)(K / 256) * (size_t)sb_bytes_of(type), type, (int)N};
 }
@@ -2436,10 +1936,12 @@ hipError_t launch_gemm(int type, const void *x, bool x_is_bf16, int64_t M, int64
     e = launch_gemm_q6(xhi, rscale, W, bias, y, M, N, K, ks, part, s);
   } else if (plan.wide == 2) {
     e = launch_gemm_pair(type, xhi, xsum, rscale, W, bias, y, M, N, K, ks, part, s);
-  } else if (plan.wide) {
+  } else if (plan.wide == 1) {
     e = launch_gemm_wide(type, xhi, xsum, rscale, W, bias, y, M, N, K, ks, part, s);
   } else {
-    e = launch_gemm_tiled(type, xhi, xsum, rscale, W, bias, y, M, N, K, plan, part, s);
+    PrefillMats mats{};
+    mats.mat[0] = PrefillMat{W, bias, y, part, n, ks, 0, 0, 0};
+    e = launch_gemm_f32(type, xhi, nullptr, xsum, rscale, M, K, mats, 1, s);
   }
   return e != hipSuccess ? e : launch_splitk_reduce(&red, 1, M, rscale, s);
 }

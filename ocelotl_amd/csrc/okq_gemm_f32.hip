@@ -1,6 +1,13 @@
 // okq_gemm_f32.hip -- prefill dequant-GEMM for f32 activations with the
 // weights dequantised in registers: Y[M,N] = X[M,K] W[N,K]^T (+bias), Q4_K,
-// Q5_K, Q6_K and Q8_0, one or several matrices that read the same X.
+// Q5_K, Q6_K and Q8_0, one or several matrices that read the same X.  bf16
+// activations (one fp16 plane: kTwo false) take it where their own kernels
+// do not pay: Q6_K grids too small for gemm_wide_q6k_kernel's tiles (us per
+// call, against weights staged through LDS: 64 x 4096 -> 14336 80 -> 34, 300 x
+// 4096 -> 14336 185 -> 100, 128 x 14336 -> 4096 61 -> 48, 33 x 4096 -> 4096 24
+// -> 22), and Q4_K / Q5_K tensors within 256 rows of 4 GiB (elsewhere the
+// kernels of okq_gemm_wide.hip and okq_gemm_pair.hip are faster: 128 x 4096 ->
+// 1024 15.6 against 19.4).
 //
 // Numerics.  A = the pre-pass's row-scaled activations as two fp16 planes,
 // x = hi + lo to 2^-22; B = the integer part of the weight, exact in fp16
@@ -128,7 +135,7 @@ struct Cur<kQ8_0> {
 
 }  // namespace
 
-template <int kType, int kNB>
+template <int kType, int kNB, bool kTwo>
 __device__ __forceinline__ void f32_body(const _Float16 *__restrict__ xhi, const _Float16 *__restrict__ xlo,
                                          const h2 *__restrict__ xsum, const float *__restrict__ rscale, int M, int K,
                                          const PrefillMats &mats) {
@@ -139,6 +146,7 @@ __device__ __forceinline__ void f32_body(const _Float16 *__restrict__ xhi, const
   constexpr int kFM = 32 * kNB;        // tile rows
   constexpr int kRW = kFM / 8;         // rows each wave copies
   constexpr int kCP = kRW / 4;         // its copy instructions per plane and stage (4 rows each)
+  constexpr int kPieces = kTwo ? 2 * kCP : kCP;
 
   // Workgroup b runs on XCD b % 8; each matrix's (slice, tile) jobs are cut
   // into eight contiguous ranges, so every XCD holds its share of every
@@ -399,12 +407,12 @@ __device__ __forceinline__ void f32_body(const _Float16 *__restrict__ xhi, const
     dequant(0, b1, b2);
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
-      {
-        const int ad = a_addr(s);
+      if (kTwo || s < 7) {  // one plane: al takes the next step's fragments
+        const int ad = a_addr(kTwo ? s : s + 1);
 #pragma unroll
-        for (int i = 0; i < kNB; ++i) al[i] = a_at(bufA + kPlane, ad, i);
+        for (int i = 0; i < kNB; ++i) al[i] = a_at(kTwo ? bufA + kPlane : bufA, ad, i);
       }
-      if (s < 2 * kCP) copy_piece(s, st_next, nbufA);
+      if (s < kPieces) copy_piece(s, st_next, nbufA);
       if (kMins && s == 7) copy_sums(st_next, nbufX);
       __builtin_amdgcn_sched_barrier(0);  // the lo reads issue ahead of the hi MFMAs
       const bool restart = kPerBlock ? (s & 1) == 0 : (h == 0 && s == 0);
@@ -417,14 +425,19 @@ __device__ __forceinline__ void f32_body(const _Float16 *__restrict__ xhi, const
 #pragma unroll
         for (int i = 0; i < kNB; ++i) accs[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i], b2, accs[i], 0, 0, 0);
       }
-      if (s < 7) {
-        const int ad = a_addr(s + 1);
+      if constexpr (kTwo) {
+        if (s < 7) {
+          const int ad = a_addr(s + 1);
 #pragma unroll
-        for (int i = 0; i < kNB; ++i) ah[i] = a_at(bufA, ad, i);
+          for (int i = 0; i < kNB; ++i) ah[i] = a_at(bufA, ad, i);
+        }
+        __builtin_amdgcn_sched_barrier(0);  // and the next hi reads ahead of the lo MFMAs
+#pragma unroll
+        for (int i = 0; i < kNB; ++i) accs[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[i], b1, accs[i], 0, 0, 0);
+      } else if (s < 7) {
+#pragma unroll
+        for (int i = 0; i < kNB; ++i) ah[i] = al[i];
       }
-      __builtin_amdgcn_sched_barrier(0);  // and the next hi reads ahead of the lo MFMAs
-#pragma unroll
-      for (int i = 0; i < kNB; ++i) accs[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[i], b1, accs[i], 0, 0, 0);
       if (s < 7) {
         dequant(s + 1, n1, n2);
         b1 = n1;
@@ -479,7 +492,7 @@ __device__ __forceinline__ void f32_body(const _Float16 *__restrict__ xhi, const
   const int last = nst - 1;
   auto clamp_st = [&](int st) { return st < last ? st : last; };
 #pragma unroll
-  for (int t = 0; t < 2 * kCP; ++t) copy_piece(t, 0, fA0);
+  for (int t = 0; t < kPieces; ++t) copy_piece(t, 0, fA0);
   if constexpr (kMins) copy_sums(0, fX0);
   if (tid < kFM) fR[tid] = m0 + tid < M ? rscale[m0 + tid] : 0.0f;
   ld_raw(0);
@@ -607,11 +620,11 @@ __device__ __forceinline__ void f32_body(const _Float16 *__restrict__ xhi, const
 }
 
 // Tiles of 32 kNB rows (a row's result does not depend on the height).
-template <int kType, int kNB>
+template <int kType, int kNB, bool kTwo>
 __global__ __launch_bounds__(512) void gemm_f32_kernel(const _Float16 *__restrict__ xhi, const _Float16 *__restrict__ xlo,
                                                        const h2 *__restrict__ xsum, const float *__restrict__ rscale,
                                                        int M, int K, PrefillMats mats) {
-  f32_body<kType, kNB>(xhi, xlo, xsum, rscale, M, K, mats);
+  f32_body<kType, kNB, kTwo>(xhi, xlo, xsum, rscale, M, K, mats);
 }
 
 // Tile height in 32-row blocks: a stage of 2, 3 or 4 blocks takes about 0.6,
@@ -644,22 +657,31 @@ hipError_t launch_gemm_f32(int type, const _Float16 *xhi, const _Float16 *xlo, c
   const dim3 grid((unsigned)(px * 8)), block(512);
   const h2 *sums = static_cast<const h2 *>(xsum);
   const int nb = tile_blocks(M);
-#define OKQ_F32(TYPE_)                                                                                                   \
+#define OKQ_F32_NB(TYPE_, TWO_)                                                                                         \
   if (nb == 2)                                                                                                          \
-    launch_timed(gemm_f32_kernel<TYPE_, 2>, grid, block, 0u, s, xhi, xlo, sums, rscale, (int)M, (int)K, mats);           \
+    launch_timed(gemm_f32_kernel<TYPE_, 2, TWO_>, grid, block, 0u, s, xhi, xlo, sums, rscale, (int)M, (int)K, mats);     \
   else if (nb == 3)                                                                                                     \
-    launch_timed(gemm_f32_kernel<TYPE_, 3>, grid, block, 0u, s, xhi, xlo, sums, rscale, (int)M, (int)K, mats);           \
+    launch_timed(gemm_f32_kernel<TYPE_, 3, TWO_>, grid, block, 0u, s, xhi, xlo, sums, rscale, (int)M, (int)K, mats);     \
   else                                                                                                                  \
-    launch_timed(gemm_f32_kernel<TYPE_, 4>, grid, block, 0u, s, xhi, xlo, sums, rscale, (int)M, (int)K, mats)
-  if (type == kQ4_K) {
-    OKQ_F32(kQ4_K);
-  } else if (type == kQ5_K) {
-    OKQ_F32(kQ5_K);
-  } else if (type == kQ6_K) {
-    OKQ_F32(kQ6_K);
-  } else {
-    OKQ_F32(kQ8_0);
+    launch_timed(gemm_f32_kernel<TYPE_, 4, TWO_>, grid, block, 0u, s, xhi, xlo, sums, rscale, (int)M, (int)K, mats)
+#define OKQ_F32(TYPE_)          \
+  if (xlo) {                    \
+    OKQ_F32_NB(TYPE_, true);    \
+  } else {                      \
+    OKQ_F32_NB(TYPE_, false);   \
   }
+  if (type == kQ4_K) {
+    OKQ_F32(kQ4_K)
+  } else if (type == kQ5_K) {
+    OKQ_F32(kQ5_K)
+  } else if (type == kQ6_K) {
+    OKQ_F32(kQ6_K)
+  } else if (xlo) {  // bf16 Q8_0: okq_gemm_q8.hip
+    OKQ_F32_NB(kQ8_0, true);
+  } else {
+    return hipErrorInvalidValue;
+  }
+#undef OKQ_F32_NB
 #undef OKQ_F32
   return hipGetLastError();
 }

@@ -3,7 +3,7 @@
 // Q5_K is the same contraction with the fifth bit of every weight taken from
 // the block's 32 qh bytes (sc * q5 <= 1953 stays an exact fp16 integer).
 //
-// Operands and numerics are those of gemm_kq_kernel (okq_gemm.hip): A = the
+// Operands and numerics (see okq_gemm.hip): A = the
 // pre-pass's row-scaled fp16 activations, B = sc * q exact in fp16, every
 // product exact, f32 accumulation; d is applied per super-block in f32.  The
 // min term  -sum_sb dmin_sb sum_j m_j xsum_j  is contracted by MFMAs straight

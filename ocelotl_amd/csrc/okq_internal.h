@@ -87,8 +87,8 @@ hipError_t launch_swiglu(const float *gate, const float *up, int64_t n, float *o
 
 // MFMA dequant-GEMM: Y[M, N] = bias + X[M, K] W[N, K]^T with X f32 or bf16.
 // How launch_gemm runs an (M, N, K) problem: tile rows, split-K factor and
-// the workspace layout (tiled kernel: activation planes, per-32 sums, row
-// scales, split-K partials; decode-batch kernel: split-K partials only),
+// the workspace layout (prefill: activation planes, per-32 sums, row scales,
+// split-K partials; decode-batch and Q8_0 bf16 kernels: split-K partials only),
 // 256-byte aligned offsets from the workspace base.
 struct GemmPlan {
   int bm;              // 32: the decode-batch kernel (M <= 32), else the tile height
@@ -96,11 +96,12 @@ struct GemmPlan {
   int kwaves;          // decode-batch kernel, unsplit K: waves that split a tile's K inside the workgroup;
                        // Q8_0 kernel: waves per workgroup (4 or 8)
   int ksplit;
-  int wide;            // weights dequantised in registers (bf16 activations): 1 the wide kernel (Q4_K / Q5_K,
-                       // 128 x 256 tiles, one workgroup per CU), 2 the pair kernel (Q4_K / Q5_K, 128 x 128
-                       // tiles, two per CU), 3 the Q8_0 kernel (128 x 128 or 128 x 256 tiles),
-                       // 4 the Q6_K kernel (128 x 256 tiles);
-                       // 5 f32 activations, every format (128 x 256 tiles)
+  int wide;            // prefill kernel (0: decode batch): 1 the wide kernel (bf16 Q4_K / Q5_K,
+                       // 128 x 256 tiles, one workgroup per CU), 2 the pair kernel (bf16 Q4_K / Q5_K, 128 x 128
+                       // tiles, two per CU), 3 the Q8_0 kernel (bf16, 128 x 128 or 128 x 256 tiles),
+                       // 4 the Q6_K kernel (bf16, 128 x 256 tiles),
+                       // 5 f32 activations, every format, 6 bf16 ones in its one-plane form
+                       // (32 gemm_f32_blocks(M) x 256 tiles)
   size_t off_lo, off_sums, off_rscale, off_part, workspace;
 };
 // Size of the allocation-free entry point's static scratch.
@@ -165,7 +166,7 @@ hipError_t launch_gemm_q8(const void *x, const void *w, const float *bias, float
                           int ksplit, int waves, float *part, hipStream_t s);
 
 // f32 activations, every linear format (okq_gemm_f32.hip): the pre-pass's two
-// fp16 planes, 128 x 256 tiles, one 8-wave workgroup per CU; up to
+// fp16 planes (xlo null: bf16 activations' one), 128 x 256 tiles, one 8-wave workgroup per CU; up to
 // kPrefillMats matrices of one format that read the same activations in one
 // launch, each with its own K split into whole super-blocks (ksplit > 1:
 // partials [ksplit][M][n] at part).

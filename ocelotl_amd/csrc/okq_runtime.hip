@@ -266,7 +266,7 @@ enum class Path { Auto, Gemv, Gemm };
 // serves up to four rows) unless the weights are large enough for the
 // streaming decode-batch MFMA kernel to repay its fixed cost (activation
 // staging, the split-K reduction launch: ~11 us); above kGemvMaxRows the MFMA
-// path always (the decode-batch kernel up to 32 rows, the tiled kernel
+// path always (the decode-batch kernel up to 32 rows, the prefill kernels
 // beyond).  Per call in graphs over HBM-resident weight copies, decode-batch
 // kernel vs GEMV (us):
 //   Q6_K 4096x14336 (48 MB): 24.2/21.3 at 2 rows, 23.5/32.0 at 3, 23.5/37.8 at 4

@@ -77,6 +77,26 @@ def test_f32_prefill_matches_float64(torch, okq, orc, t, rows, k, n):
     assert bool((err <= bound).all()), float((err / bound).max())
 
 
+@pytest.mark.parametrize("rows,k,n", [(33, 256, 40), (64, 768, 255), (65, 2304, 257), (97, 512, 520), (128, 4096, 300),
+                                      (333, 1024, 512)])
+def test_bf16_q6k_prefill_on_small_grids_matches_float64(torch, okq, orc, rows, k, n):
+    """bf16 activations through Q6_K grids that do not fill the 8-wave tiles:
+    the one-plane form.  Every product is exact; the sums of at most 2 K / 16
+    accumulations are bounded as above."""
+    print(f"[gpu] bf16 Q6_K prefill rows={rows} K={k} N={n}", flush=True)
+    wq = orc.quantize(O.Q6_K, orc.normal(9300 + k, n * k, 0.02))
+    x = _dev(torch, orc.normal(9301 + rows, rows * k, 1.0)).view(rows, k).to(torch.bfloat16)
+    x[:, :3] *= 100.0
+    wd, bd = _dev(torch, wq), _dev(torch, orc.normal(9302, n, 0.1))
+    out = _linear(torch, okq, O.Q6_K, x, rows, k, wd, n, bd, entry="okq_linear_out_by_in_q_bf16")
+    torch.cuda.synchronize()
+    w = _dev(torch, orc.dequantize(O.Q6_K, wq, n * k)).view(n, k).double()
+    want = x.double() @ w.t() + bd.double()
+    bound = 2.0 ** -20 * x.double().abs().sum(1, keepdim=True) * 2 * w.abs().amax(1) + 2.0 ** -22 * want.abs()
+    err = (out.view(rows, n).double() - want).abs()
+    assert bool((err <= bound).all()), float((err / bound).max())
+
+
 @pytest.mark.parametrize("types,rows,k,ns", [
     ([O.Q4_K, O.Q4_K, O.Q6_K], 70, 4096, [1024, 256, 256]),
     ([O.Q8_0, O.Q8_0, O.Q8_0], 333, 2048, [2048, 512, 300]),
