@@ -70,6 +70,12 @@ __device__ __forceinline__ void load8(const void *X, int64_t base, float v[8]) {
   }
 }
 
+__device__ __forceinline__ void put8(float *p, int64_t base, const float v[8]) {
+  float4 *o = reinterpret_cast<float4 *>(p + base);
+  o[0] = float4{v[0], v[1], v[2], v[3]};
+  o[1] = float4{v[4], v[5], v[6], v[7]};
+}
+
 // Shared by both forms of the pre-pass: the row's scale from its max |x|,
 // then the scaled fp16 planes and per-32 sums of 8 values (one chunk; fixed
 // order: pairs within a thread, then the four threads of the run through DPP).
@@ -175,7 +181,7 @@ __device__ __forceinline__ float x_at(const void *X, int64_t i) {
 __device__ __forceinline__ bool non_finite(float v) { return !(fabsf(v) <= 3.4028235e38f); }
 
 template <bool kF32>
-__device__ void prep_ieee_row(const void *__restrict__ X, int m, int K, const PrepIeees &Ps, int tid) {
+__device__ void prep_ieee_row(const void *X, int m, int K, const PrepIeees &Ps, int tid) {
   __shared__ int cnt;
   __shared__ int pos[kIeeeCap];
   if (tid == 0) cnt = 0;
@@ -210,11 +216,17 @@ __device__ void prep_ieee_row(const void *__restrict__ X, int m, int K, const Pr
 // CH > 0: each thread holds its CH chunks of 8 activations in registers
 // (chunk c = tid + 256 i), so the row is read once; CH == 0: rows longer than
 // 8 chunks per thread are read twice (max, then convert).
-template <bool kF32, int CH>
-__global__ __launch_bounds__(256) void gemm_prep_kernel(const void *__restrict__ X, int M, int K,
-                                                        _Float16 *__restrict__ xhi, _Float16 *__restrict__ xlo,
-                                                        h2 *__restrict__ xsum, float *__restrict__ rscale,
-                                                        PrepIeees ieee) {
+//
+// kPro (f32, CH > 0) forms the activations on the way, so that they are not
+// written and read once more ahead of the pre-pass: the RMSNorm of X with
+// weight pro.a, or silu(X) * pro.a, which is also left in pro.out (X itself
+// may be that buffer).  333 rows x 4096: RMSNorm and pre-pass 10.4 us, together
+// 5.4; 512 rows x 14336: SwiGLU and pre-pass 27.7 us, together 21.3.
+template <bool kF32, int CH, int kPro>
+__global__ __launch_bounds__(256) void gemm_prep_kernel(const void *X, int M, int K, _Float16 *__restrict__ xhi,
+                                                        _Float16 *__restrict__ xlo, h2 *__restrict__ xsum,
+                                                        float *__restrict__ rscale, PrepIeees ieee, PrepPro pro) {
+  static_assert(kPro == kProNone || (kF32 && CH > 0), "the neighbours take f32 rows held in registers");
   __shared__ uint32_t red[4];
   const int m = (int)blockIdx.x;
   const int tid = (int)threadIdx.x;
@@ -233,6 +245,45 @@ __global__ __launch_bounds__(256) void gemm_prep_kernel(const void *__restrict__
         for (int e = 0; e < 8; ++e) v[i][e] = 0.0f;
       }
     }
+    if constexpr (kPro == kProRms) {
+      // the reference's order per value (crates/kernels/src/rmsnorm.rs:116-128)
+      float ss = 0.0f;
+#pragma unroll
+      for (int i = 0; i < CH; ++i)
+#pragma unroll
+        for (int e = 0; e < 8; e += 4)
+          ss += (v[i][e] * v[i][e] + v[i][e + 1] * v[i][e + 1]) + (v[i][e + 2] * v[i][e + 2] + v[i][e + 3] * v[i][e + 3]);
+      float w[CH][8];
+#pragma unroll
+      for (int i = 0; i < CH; ++i) {
+        const int c = tid + 256 * i;
+        load8<true>(pro.a, 8 * (int64_t)(c < chunks ? c : 0), w[i]);
+      }
+      __shared__ float sq[4];
+      ss = wave_sum(ss);
+      if ((tid & 63) == 0) sq[tid >> 6] = ss;
+      __syncthreads();
+      const float inv = 1.0f / sqrtf(((sq[0] + sq[1]) + (sq[2] + sq[3])) / (float)K + pro.eps);
+#pragma unroll
+      for (int i = 0; i < CH; ++i)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[i][e] = v[i][e] * inv * w[i][e];
+    } else if constexpr (kPro == kProSwiGLU) {
+#pragma unroll
+      for (int i = 0; i < CH; ++i) {
+        const int c = tid + 256 * i;
+        if (c < chunks) {
+          float u[8];
+          load8<true>(pro.a, row + 8 * (int64_t)c, u);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float sig = 1.0f / (1.0f + expf(-v[i][e]));
+            v[i][e] = (v[i][e] * sig) * u[e];
+          }
+          put8(pro.out, row + 8 * (int64_t)c, v[i]);
+        }
+      }
+    }
 #pragma unroll
     for (int i = 0; i < CH; ++i)
 #pragma unroll
@@ -246,7 +297,16 @@ __global__ __launch_bounds__(256) void gemm_prep_kernel(const void *__restrict__
       const int c = tid + 256 * i;  // chunks is a multiple of 32: runs never straddle the bound
       prep_chunk<kF32>(v[i], s, c < chunks, row + 8 * (int64_t)c, m, K, c, tid, xhi, xlo, xsum);
     }
-    if (bad) prep_ieee_row<kF32>(X, m, K, ieee, tid);
+    if (bad) {
+      if constexpr (kPro == kProRms) {  // the IEEE row reads finished activations
+#pragma unroll
+        for (int i = 0; i < CH; ++i) {
+          const int c = tid + 256 * i;
+          if (c < chunks) put8(pro.out, row + 8 * (int64_t)c, v[i]);
+        }
+      }
+      prep_ieee_row<kF32>(kPro == kProNone ? X : (const void *)pro.out, m, K, ieee, tid);
+    }
     return;
   }
   // pass 1: row max |x|
@@ -1285,15 +1345,17 @@ struct ReduceMat {
   float *y;
   int n, ks, bx0;  // outputs, slices, first column block
 };
+template <bool kOne>
 struct ReduceMats {
-  ReduceMat mat[kPrefillMats];
+  ReduceMat mat[kOne ? 1 : kPrefillMats];
 };
 template <int KB, int RR, bool kOne>
-__global__ __launch_bounds__(256) void splitk_reduce4_kernel(ReduceMats mats, int M, const float *__restrict__ rscale) {
+__global__ __launch_bounds__(256) void splitk_reduce4_kernel(ReduceMats<kOne> mats, int M,
+                                                             const float *__restrict__ rscale) {
   const int bx = (int)blockIdx.x;
-  const int mi = kOne ? 0
-                      : (int)(bx >= sarg(mats.mat[1].bx0)) + (int)(bx >= sarg(mats.mat[2].bx0)) +
-                            (int)(bx >= sarg(mats.mat[3].bx0));
+  int mi = 0;
+  if constexpr (!kOne)
+    mi = (int)(bx >= sarg(mats.mat[1].bx0)) + (int)(bx >= sarg(mats.mat[2].bx0)) + (int)(bx >= sarg(mats.mat[3].bx0));
   const ReduceMat &mt = mats.mat[mi];
   auto arg = [](auto v) {  // fields at a computed index come in one batch of scalar loads
     if constexpr (kOne) return v;
@@ -1355,7 +1417,7 @@ __global__ __launch_bounds__(256) void splitk_reduce4_kernel(ReduceMats mats, in
 static hipError_t launch_splitk_reduce(const ReduceMat *m, int count, int64_t M, const float *rscale, hipStream_t s) {
   constexpr int RR = kReduceRows;
   const bool rows_fit = (M + RR - 1) / RR <= 65535;
-  ReduceMats rm{};
+  ReduceMats<false> rm{};
   int c = 0, bx = 0, kmax = 0;
   for (int i = 0; i < count; ++i) {
     if (m[i].ks <= 1) continue;
@@ -1377,8 +1439,9 @@ static hipError_t launch_splitk_reduce(const ReduceMat *m, int count, int64_t M,
   if (c == 0) return hipSuccess;
   for (int i = c; i < kPrefillMats; ++i) rm.mat[i].bx0 = INT32_MAX;
   const dim3 g4((unsigned)bx, (unsigned)((M + RR - 1) / RR));
+  const ReduceMats<true> rm1{{rm.mat[0]}};
 #define OKQ_REDUCE(KB_)                                                                                              \
-  if (c == 1) hipLaunchKernelGGL((splitk_reduce4_kernel<KB_, RR, true>), g4, dim3(256), 0, s, rm, (int)M, rscale);  \
+  if (c == 1) hipLaunchKernelGGL((splitk_reduce4_kernel<KB_, RR, true>), g4, dim3(256), 0, s, rm1, (int)M, rscale);  \
   else hipLaunchKernelGGL((splitk_reduce4_kernel<KB_, RR, false>), g4, dim3(256), 0, s, rm, (int)M, rscale)
   if (kmax <= 2) {
     OKQ_REDUCE(2);
@@ -1840,23 +1903,42 @@ static PrepIeee prep_ieee(int type, int64_t K, const void *w, int64_t N, const f
 
 template <bool kF32>
 static hipError_t launch_prep(const void *x, int64_t M, int64_t K, _Float16 *xhi, _Float16 *xlo, h2 *xsum, float *rscale,
-                              const PrepIeees &ieee, hipStream_t s) {
+                              const PrepIeees &ieee, const PrepPro &pro, hipStream_t s) {
   // chunks of 8 activations per thread: 2 (K <= 4096), 4, 8 held in registers, longer rows read twice
   const int64_t per_thread = (K / 8 + 255) / 256;
-#define OKQ_PREP(CH_)                                                                                                 \
-  hipLaunchKernelGGL((gemm_prep_kernel<kF32, CH_>), dim3((unsigned)M), dim3(256), 0, s, x, (int)M, (int)K, xhi, xlo,  \
-                     xsum, rscale, ieee)
-  if (per_thread <= 2) OKQ_PREP(2);
-  else if (per_thread <= 4) OKQ_PREP(4);
-  else if (per_thread <= 8) OKQ_PREP(8);
-  else OKQ_PREP(0);
+#define OKQ_PREP(CH_, PRO_)                                                                                          \
+  hipLaunchKernelGGL((gemm_prep_kernel<kF32, CH_, PRO_>), dim3((unsigned)M), dim3(256), 0, s, x, (int)M, (int)K, xhi, \
+                     xlo, xsum, rscale, ieee, pro)
+#define OKQ_PREP_CH(PRO_)                     \
+  if (per_thread <= 2) OKQ_PREP(2, PRO_);     \
+  else if (per_thread <= 4) OKQ_PREP(4, PRO_); \
+  else OKQ_PREP(8, PRO_)
+  if (per_thread > 8) {
+    if (pro.kind != kProNone) return hipErrorInvalidValue;  // callers check prep_folds
+    OKQ_PREP(0, kProNone);
+    return hipGetLastError();
+  }
+  if constexpr (kF32) {
+    if (pro.kind == kProRms) {
+      OKQ_PREP_CH(kProRms);
+      return hipGetLastError();
+    }
+    if (pro.kind == kProSwiGLU) {
+      OKQ_PREP_CH(kProSwiGLU);
+      return hipGetLastError();
+    }
+  }
+  OKQ_PREP_CH(kProNone);
+#undef OKQ_PREP_CH
 #undef OKQ_PREP
   return hipGetLastError();
 }
 
+bool prep_folds(int64_t K) { return K <= 8 * 8 * 256; }
+
 hipError_t launch_prefill_multi(const void *x, int64_t M, int64_t K, int count, const int *types, const void *const *w,
                                 const int64_t *N, const float *const *bias, float *const *y, void *workspace,
-                                const PrefillPlan &plan, hipStream_t s) {
+                                const PrefillPlan &plan, hipStream_t s, const PrepPro &pro) {
   if (count < 1 || count > kPrefillMats || plan.base.wide != 5) return hipErrorInvalidValue;
   char *ws = static_cast<char *>(workspace);
   _Float16 *xhi = reinterpret_cast<_Float16 *>(ws), *xlo = reinterpret_cast<_Float16 *>(ws + plan.base.off_lo);
@@ -1871,7 +1953,7 @@ hipError_t launch_prefill_multi(const void *x, int64_t M, int64_t K, int count, 
     red[i] = ReduceMat{reinterpret_cast<float *>(ws + plan.off_part[i]), bias[i], y[i], (int)N[i], ks, 0};
   }
   ieee.count = count;
-  hipError_t e = launch_prep<true>(x, M, K, xhi, xlo, xsum, rscale, ieee, s);
+  hipError_t e = launch_prep<true>(x, M, K, xhi, xlo, xsum, rscale, ieee, pro, s);
   // one launch per format, over its matrices
   bool done[kPrefillMats] = {};
   for (int i = 0; i < count && e == hipSuccess; ++i) {
@@ -1916,7 +1998,7 @@ hipError_t launch_gemm(int type, const void *x, bool x_is_bf16, int64_t M, int64
     g.base = plan;
     g.ksplit[0] = ks;
     g.off_part[0] = plan.off_part;
-    return launch_prefill_multi(x, M, K, 1, &type, &w, &N, &bias, &y, workspace, g, s);
+    return launch_prefill_multi(x, M, K, 1, &type, &w, &N, &bias, &y, workspace, g, s, PrepPro{});
   }
   if (plan.wide == 3) {
     if (!x_is_bf16 || type != kQ8_0) return hipErrorInvalidValue;
@@ -1930,7 +2012,7 @@ hipError_t launch_gemm(int type, const void *x, bool x_is_bf16, int64_t M, int64
   PrepIeees ieee{};
   ieee.mat[0] = prep_ieee(type, K, W, N, bias, y);
   ieee.count = 1;
-  hipError_t e = launch_prep<false>(x, M, K, xhi, nullptr, xsum, rscale, ieee, s);
+  hipError_t e = launch_prep<false>(x, M, K, xhi, nullptr, xsum, rscale, ieee, PrepPro{}, s);
   if (e != hipSuccess) return e;
   if (plan.wide == 4) {
     e = launch_gemm_q6(xhi, rscale, W, bias, y, M, N, K, ks, part, s);

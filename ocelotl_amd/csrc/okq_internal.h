@@ -192,10 +192,21 @@ struct PrefillPlan {
   int ksplit[kPrefillMats];
   size_t off_part[kPrefillMats], workspace;
 };
+// What the pre-pass forms from x first (kind: GemvProKind): nothing, the
+// RMSNorm of x with weight a (out: scratch [M][K], written for rows holding
+// infinities or NaNs), or silu(x) * a, also written to out (x itself may be
+// it).  prep_folds: the row lengths that it can do so for.
+struct PrepPro {
+  int kind;
+  const float *a;
+  float eps;
+  float *out;
+};
+bool prep_folds(int64_t K);
 PrefillPlan prefill_plan(int64_t M, int64_t K, int count, const int *types, const int64_t *N, int cu_count);
 hipError_t launch_prefill_multi(const void *x, int64_t M, int64_t K, int count, const int *types, const void *const *w,
                                 const int64_t *N, const float *const *bias, float *const *y, void *workspace,
-                                const PrefillPlan &plan, hipStream_t s);
+                                const PrefillPlan &plan, hipStream_t s, const PrepPro &pro);
 hipError_t launch_gemm_f32(int type, const _Float16 *xhi, const _Float16 *xlo, const void *xsum, const float *rscale,
                            int64_t M, int64_t K, PrefillMats &mats, int count, hipStream_t s);
 

@@ -583,15 +583,23 @@ okq_status okq_linear_out_by_in_q_bf16(const uint16_t *x, int64_t rows, int64_t 
 // More than 32 f32 rows through `count` MFMA-routed matrices (the stream's
 // enqueue lock held): bit for bit each matrix's own call.  Where the shared
 // workspace cannot be had (a capture before any call of this size), the
-// matrices run one by one, each within the workspace of its own call.
+// matrices run one by one, each within the workspace of its own call, after
+// `pro` as a pass of its own.
 static okq_status prefill_multi(const float *x, int64_t rows, int64_t K, int count, const int *types,
                                 const void *const *w, const int64_t *N, const float *const *bias, float *const *out,
-                                hipStream_t s, int dev, const DevInfo &info) {
+                                hipStream_t s, int dev, const DevInfo &info,
+                                const okq::PrepPro &pro = okq::PrepPro{}) {
   const okq::PrefillPlan plan = okq::prefill_plan(rows, K, count, types, N, info.cu_count);
   void *ws = nullptr;
   if (get_workspace(dev, s, plan.workspace, &ws) == OKQ_OK)
-    return hip_status(okq::launch_prefill_multi(x, rows, K, count, types, w, N, bias, out, ws, plan, s),
+    return hip_status(okq::launch_prefill_multi(x, rows, K, count, types, w, N, bias, out, ws, plan, s, pro),
                       "grouped gemm launch");
+  if (pro.kind != okq::kProNone) {
+    const hipError_t e = pro.kind == okq::kProRms ? okq::launch_rmsnorm(x, rows, K, pro.a, pro.eps, pro.out, s)
+                                                  : okq::launch_swiglu(x, pro.a, rows * K, pro.out, s);
+    if (e != hipSuccess) return hip_status(e, "neighbour launch");
+    x = pro.out;
+  }
   for (int i = 0; i < count; ++i) {
     const okq::GemmPlan p = okq::gemm_plan(types[i], rows, N[i], K, false, info.cu_count);
     okq_status st = get_workspace(dev, s, p.workspace, &ws);
@@ -906,6 +914,27 @@ okq_status okq_rmsnorm_linear_q_multi(const float *x, int64_t rows, int64_t hidd
   st = get_workspace(dev, s, (size_t)rows * (size_t)hidden * sizeof(float), &ws, 1);
   if (st != OKQ_OK) return st;
   float *xn = static_cast<float *>(ws);
+  if (rows > okq::kGemmDecodeRows && okq::prep_folds(hidden)) {
+    // prefill: the GEMM's pre-pass normalises the rows as it reads them
+    int types[okq::kGemvMaxProblems], c = 0;
+    const void *mw[okq::kGemvMaxProblems];
+    int64_t mn[okq::kGemvMaxProblems];
+    const float *mb[okq::kGemvMaxProblems];
+    float *mo[okq::kGemvMaxProblems];
+    bool all = true;
+    for (int i = 0; i < count; ++i) {
+      if (out_features[i] == 0) continue;
+      all = all && okq::gemm_supported((int)w_type, rows, hidden, out_features[i]);
+      types[c] = (int)w_type;
+      mw[c] = w[i];
+      mn[c] = out_features[i];
+      mb[c] = b[i];
+      mo[c++] = out[i];
+    }
+    if (all)
+      return prefill_multi(x, rows, hidden, c, types, mw, mn, mb, mo, s, dev, info,
+                           okq::PrepPro{okq::kProRms, norm_weight, epsilon, xn});
+  }
   hipError_t e = okq::launch_rmsnorm(x, rows, hidden, norm_weight, epsilon, xn, s);
   if (e != hipSuccess) return hip_status(e, "rmsnorm launch");
   // the normalised rows then go through the grouped dispatch of okq_gemv_multi
@@ -1004,6 +1033,15 @@ okq_status okq_mlp_gated_silu_q(const float *x, int64_t rows, int64_t hidden, in
       if (e != hipSuccess) return hip_status(e, "mlp down launch");
     }
     return ok();
+  }
+  if (rows > okq::kGemmDecodeRows && okq::prep_folds(intermediate) &&
+      okq::gemm_supported((int)down_type, rows, intermediate, hidden)) {
+    // prefill: the down GEMM's pre-pass forms silu(gate) * up as it reads them
+    const int type = (int)down_type;
+    const int64_t n = hidden;
+    const float *nob = nullptr;
+    return prefill_multi(gate_buf, rows, intermediate, 1, &type, &down_w, &n, &nob, &out, s, dev, info,
+                         okq::PrepPro{okq::kProSwiGLU, up_buf, 0.0f, gate_buf});
   }
   if (!swiglu_done) {
     hipError_t e = okq::launch_swiglu(gate_buf, up_buf, rows * intermediate, gate_buf, s);

@@ -157,3 +157,89 @@ def test_f32_prefill_near_the_static_scratch(torch, okq, orc):
     b = _linear(torch, okq, t, xd, rows, k, wd, n)
     torch.cuda.synchronize()
     assert (a.cpu().numpy().view(np.uint32) == b.cpu().numpy().view(np.uint32)).all()
+
+
+@pytest.mark.parametrize("t,rows,hidden,ns", [
+    (O.Q4_K, 40, 256, [64, 17]),           # the last thread's chunks past the row
+    (O.Q8_0, 333, 4096, [512, 128, 128]),
+    (O.Q6_K, 34, 8192, [96]),              # four chunks per thread
+    (O.Q5_K, 33, 16384, [40, 8]),          # eight
+    (O.Q4_K, 33, 16640, [40]),             # longer rows: normalised by a pass of its own
+])
+def test_rmsnorm_in_the_prepass_matches_float64(torch, okq, orc, t, rows, hidden, ns):
+    """okq_rmsnorm_linear_q_multi above 32 rows.  The normalised row carries a
+    relative error of fewer than 2^-18 (a tree of under 40 roundings in the
+    sum, a square root, a division, two products), the linear the bound of
+    test_f32_prefill_matches_float64.  A row with an infinity is NaN
+    throughout (inf * (1 / inf))."""
+    print(f"[gpu] rms prepass type={t} rows={rows} hidden={hidden} N={ns}", flush=True)
+    x = orc.normal(9400 + hidden, rows * hidden, 1.5).reshape(rows, hidden)
+    x[1, 3] = np.inf
+    g = orc.normal(9401 + hidden, hidden, 1.0)
+    xd, gd = _dev(torch, x), _dev(torch, g)
+    wds = [_dev(torch, orc.quantize(t, orc.normal(9410 + i, n * hidden, 0.02))) for i, n in enumerate(ns)]
+    outs = [torch.full((rows * n,), 7.0, device="cuda") for n in ns]
+    arr = lambda ty, vals: (ty * len(ns))(*vals)
+    okq.call("okq_rmsnorm_linear_q_multi", xd.data_ptr(), rows, hidden, gd.data_ptr(), 1e-6, t, len(ns),
+             arr(ctypes.c_void_p, [w.data_ptr() for w in wds]), arr(ctypes.c_uint64, [w.numel() for w in wds]),
+             arr(ctypes.c_int64, ns), None, arr(ctypes.c_void_p, [o.data_ptr() for o in outs]),
+             torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    x64 = xd.double()
+    xn = x64 / torch.sqrt((x64 * x64).mean(1, keepdim=True) + float(np.float32(1e-6))) * gd.double()
+    keep = torch.arange(rows, device="cuda") != 1
+    for n, w, o in zip(ns, wds, outs):
+        got = o.view(rows, n).double()
+        wm = _dev(torch, orc.dequantize(t, w.cpu().numpy(), n * hidden)).view(n, hidden).double()
+        want = xn[keep] @ wm.t()
+        mag = xn[keep].abs().sum(1, keepdim=True) * wm.abs().amax(1)
+        assert bool(((got[keep] - want).abs() <= (2.0 ** -19 + 2.0 ** -18) * mag).all())
+        assert bool(torch.isnan(got[1]).all())
+
+
+@pytest.mark.parametrize("t,td,rows,hidden,inter", [
+    (O.Q4_K, O.Q6_K, 40, 1024, 2816), (O.Q8_0, O.Q4_K, 130, 512, 8192), (O.Q6_K, O.Q8_0, 33, 768, 16640),
+])
+def test_swiglu_in_the_prepass_leaves_its_rows(torch, okq, orc, t, td, rows, hidden, inter):
+    """okq_mlp_gated_silu_q above 32 rows: gate_buf holds silu(g) * u of the
+    grouped projections (up to the rounding of exp), up_buf their u bit for
+    bit, and out is okq_linear_out_by_in_q on gate_buf bit for bit -- also in a
+    row with an infinity, and captured on a stream without workspaces of this
+    size but those of the single calls."""
+    print(f"[gpu] swiglu prepass types={t},{td} rows={rows} hidden={hidden} inter={inter}", flush=True)
+    x = orc.normal(9500 + rows, rows * hidden, 1.0).reshape(rows, hidden)
+    x[2, 1] = -np.inf
+    xd = _dev(torch, x)
+    gd, ud, dd = (_dev(torch, orc.quantize(ty, orc.normal(9501 + i, n * k, 0.02)))
+                  for i, (ty, n, k) in enumerate([(t, inter, hidden), (t, inter, hidden), (td, hidden, inter)]))
+    gb, ub, out = (torch.full((rows * n,), 7.0, device="cuda") for n in (inter, inter, hidden))
+    s = torch.cuda.current_stream().cuda_stream
+    args = (xd.data_ptr(), rows, hidden, inter, t, gd.data_ptr(), gd.numel(), t, ud.data_ptr(), ud.numel(), td,
+            dd.data_ptr(), dd.numel(), gb.data_ptr(), ub.data_ptr(), out.data_ptr())
+    okq.call("okq_mlp_gated_silu_q", *args, s)
+    g = _linear(torch, okq, t, xd, rows, hidden, gd, inter).cpu().numpy()
+    u = _linear(torch, okq, t, xd, rows, hidden, ud, inter).cpu().numpy()
+    down = _linear(torch, okq, td, gb, rows, inter, dd, hidden)
+    torch.cuda.synchronize()
+    same = lambda a, b: ((a.view(np.uint32) == b.view(np.uint32)) | (np.isnan(a) & np.isnan(b))).all()
+    h, got = gb.cpu().numpy(), out.cpu().numpy()
+    assert same(ub.cpu().numpy(), u) and same(got, down.cpu().numpy())
+    with np.errstate(all="ignore"):
+        want = (g * (np.float32(1.0) / (np.float32(1.0) + np.exp(-g)))) * u
+        fine = np.isfinite(want)
+        assert np.all(np.abs(h[fine] - want[fine]) <= 8 * np.spacing(np.abs(want[fine])))
+    assert (np.isfinite(h) == fine).all()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    _linear(torch, okq, t, xd, rows, hidden, gd, inter, stream=side.cuda_stream)
+    _linear(torch, okq, td, gb, rows, inter, dd, hidden, stream=side.cuda_stream)
+    side.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        okq.call("okq_mlp_gated_silu_q", *args, side.cuda_stream)
+    for _ in range(3):
+        gb.fill_(7.0)
+        out.fill_(7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert same(gb.cpu().numpy(), h) and same(out.cpu().numpy(), got)
