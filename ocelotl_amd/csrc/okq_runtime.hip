@@ -238,8 +238,10 @@ okq_status get_workspace(int dev, hipStream_t s, size_t bytes, void **out, int s
                 bytes);
   const size_t want = bytes + bytes / 2;
   void *p = nullptr;
-  if (hipMalloc(&p, want) != hipSuccess)
+  if (hipMalloc(&p, want) != hipSuccess) {
+    (void)hipGetLastError();  // callers go on with a smaller workspace: the next launch check must not see this error
     return fail(OKQ_E_ALLOC, "hip-gfx950: hipMalloc of a %zu-byte GEMM workspace failed", want);
+  }
   w.ptr = p;  // the previous buffer (if any) stays allocated: see above
   w.bytes = want;
   *out = w.ptr;
