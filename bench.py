@@ -523,7 +523,7 @@ def run_q5k(ctx: Ctx, args):
     """Q5_K, the linear path's fourth format, at the Llama-3-8B MLP shapes:
     the gate+up pair (2 x 14336x4096) as one okq_gemv_multi call at batch 1
     (the grouped GEMV launch) and at 8 rows (one decode-batch launch), and the
-    M=512 gate prefill call with bf16 activations (pre-pass + tiled kernel).
+    M=512 gate prefill call with bf16 activations (pre-pass + wide kernel).
     Each rotates over >= 512 MB of weight replicas inside a HIP graph."""
     torch = ctx.torch
     n, k = 14336, 4096

@@ -160,7 +160,7 @@ okq_status okq_linear_out_by_in_q_bf16(const uint16_t *x, int64_t rows, int64_t 
  * allocation.  Limits: a problem whose scratch exceeds 64 MiB fails with
  * OKQ_E_SHAPE before anything launches (f32 activations: every Llama-3-8B
  * shape up to 32 rows, the 128256 x 4096 output head included, whose 32-row
- * split-K partials take 62.6 MiB; the tiled GEMM while 2 x rows x
+ * split-K partials take 62.6 MiB; the prefill GEMM while 2 x rows x
  * in_features x 2 bytes plus its sums and partials fit); every call on one device
  * shares the array and keeps the last call's contents, so calls that overlap
  * on one device (several streams or threads at once) race.  The array's

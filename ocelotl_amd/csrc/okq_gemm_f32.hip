@@ -18,7 +18,7 @@
 // d is applied in f32 per super-block (Q8_0: per block of 32), with the
 // Q4_K / Q5_K min term dmin * sum_j m_j xsum_j from one more MFMA.
 //
-// Per call, against the tiled kernel that staged dequantised weights in LDS
+// Per call, against a kernel that staged dequantised weights in LDS
 // (us): 512 x 4096 -> 14336 Q4_K 219 -> 123, Q5_K 244 -> 136, Q6_K 306 -> 168,
 // Q8_0 219 -> 152; 2048 x 14336 -> 4096 Q4_K 767 -> 450, Q6_K 1007 -> 602;
 // 64 x 14336 -> 4096 Q4_K 58 -> 34; 33 x 4096 -> 4096 Q4_K 24 -> 20.
