@@ -115,7 +115,9 @@ hipError_t launch_gemm(int type, const void *x, bool x_is_bf16, int64_t M, int64
 // in one decode-batch launch (plan: gemm_plan with N = sum of the matrices'
 // rows rounded up to 16 each, which must pick the decode-batch kernel).
 // swiglu (two matrices of equal rows, gate then up): when the plan splits K,
-// the reduction leaves up in y[1] and silu(gate) * up in y[0].
+// the reduction leaves up in y[1] and silu(gate) * up in y[0]; when it does
+// not, the kernel does so where gemm_decode_pairs (f32 x, no bias).
+bool gemm_decode_pairs(const GemmPlan &plan);
 constexpr int kDecMats = 4;
 constexpr int kGemmDecodeRows = 32;  // batches up to this many rows take the decode-batch kernel
 hipError_t launch_gemm_decode_multi(int type, const void *x, bool x_is_bf16, int64_t M, int64_t K, int count,

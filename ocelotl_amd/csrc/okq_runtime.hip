@@ -624,8 +624,9 @@ static okq_status prefill_multi(const float *x, int64_t rows, int64_t K, int cou
 // the reference rule rather than bit for bit.  A single MFMA matrix, or
 // larger batches, run through okq_linear_out_by_in_q's own dispatch.
 // swiglu_pair (count 2: gate then up of a gated-SiLU MLP): when both take one
-// decode-batch launch that splits K, its reduction also applies the SiLU
-// (out[0] = silu(gate) * up, out[1] = up) and *swiglu_done says so.
+// decode-batch launch, its K split's reduction, or the launch itself where its
+// tiles go in pairs (gemm_decode_pairs), also applies the SiLU (out[0] =
+// silu(gate) * up, out[1] = up) and *swiglu_done says so.
 static okq_status grouped_linear(const float *x, int64_t rows, int64_t in_features, uint32_t w_type, int count,
                           const void *const *w, const uint64_t *w_bytes, const int64_t *out_features,
                           const float *const *b, float *const *out, void *stream, int dev, const DevInfo &info,
@@ -665,7 +666,8 @@ static okq_status grouped_linear(const float *x, int64_t rows, int64_t in_featur
     void *ws = nullptr;
     st = get_workspace(dev, s, plan.workspace, &ws);
     if (st != OKQ_OK) return st;
-    const bool swiglu = swiglu_pair && count == 2 && mfma == 2 && plan.ksplit > 1;
+    const bool swiglu =
+        swiglu_pair && count == 2 && mfma == 2 && (plan.ksplit > 1 || okq::gemm_decode_pairs(plan));
     st = hip_status(okq::launch_gemm_decode_multi((int)w_type, x, false, rows, in_features, mfma, mw, mn, mb, mo, ws,
                                                   plan, s, swiglu),
                     "gemv_multi decode-batch launch");
@@ -979,8 +981,8 @@ okq_status okq_mlp_gated_silu_q(const float *x, int64_t rows, int64_t hidden, in
   hipStream_t s = static_cast<hipStream_t>(stream);
   std::lock_guard<std::recursive_mutex> enqueue(stream_lock(dev, s));
   // gate and up: grouped like okq_gemv_multi when they share a format (one
-  // GEMV pass over both weights, or one decode-batch launch, whose split-K
-  // reduction then applies the SiLU too)
+  // GEMV pass over both weights, or one decode-batch launch, which or
+  // whose split-K reduction then applies the SiLU too)
   bool swiglu_done = false;
   // one row, a down weight that streams: gate and up row by row in pairs, so
   // that their launch also leaves silu(gate) * up in the neighbours' workspace

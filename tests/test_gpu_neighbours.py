@@ -343,6 +343,46 @@ def test_mlp_gated_silu_q_split_reduction_applies_silu(torch, okq, orc, tgu, td,
     assert (out.cpu().numpy().view(np.uint32) == out2.cpu().numpy().view(np.uint32)).all()
 
 
+@pytest.mark.parametrize("tgu,td,rows,hidden,inter", [
+    # gate and up in one decode-batch launch with unsplit K: 8, 4 and 2 tile
+    # slots per workgroup, uneven pairs per workgroup, a cut last tile
+    (O.Q4_K, O.Q6_K, 8, 4096, 14336), (O.Q4_K, O.Q4_K, 12, 1024, 8448), (O.Q5_K, O.Q4_K, 16, 1024, 7936),
+    (O.Q6_K, O.Q4_K, 9, 1280, 2816), (O.Q8_0, O.Q8_0, 10, 2048, 2600), (O.Q4_K, O.Q8_0, 13, 1024, 4096),
+])
+def test_mlp_gated_silu_q_paired_tiles_apply_silu(torch, okq, orc, tgu, td, rows, hidden, inter):
+    """As above where gate+up keep K inside the workgroup: the launch itself
+    leaves silu(gate(x)) * up(x) in gate_buf, and up(x) in up_buf bit for bit;
+    a row with an infinity holds the SiLU of its IEEE outputs."""
+    inter = inter // 32 * 32
+    print(f"[gpu] mlp paired tiles types={tgu},{td} rows={rows} hidden={hidden} inter={inter}", flush=True)
+    x = orc.normal(7600 + rows, rows * hidden, 1.0).reshape(rows, hidden)
+    x[3, 5] = np.inf
+    gd, ud, dd, xd = (_dev(torch, a) for a in (
+        orc.quantize(tgu, orc.normal(7601, inter * hidden, 0.02)),
+        orc.quantize(tgu, orc.normal(7602, inter * hidden, 0.02)),
+        orc.quantize(td, orc.normal(7603, hidden * inter, 0.02)), x))
+    gb, ub, g2, u2 = (torch.full((rows * inter,), 7.0, device="cuda") for _ in range(4))
+    out, out2 = (torch.full((rows * hidden,), 7.0, device="cuda") for _ in range(2))
+    okq.call("okq_mlp_gated_silu_q", xd.data_ptr(), rows, hidden, inter, tgu, gd.data_ptr(), gd.numel(),
+             tgu, ud.data_ptr(), ud.numel(), td, dd.data_ptr(), dd.numel(), gb.data_ptr(), ub.data_ptr(),
+             out.data_ptr(), _stream(torch))
+    okq.call("okq_gemv_multi", xd.data_ptr(), rows, hidden, tgu, 2, (ctypes.c_void_p * 2)(gd.data_ptr(), ud.data_ptr()),
+             (ctypes.c_uint64 * 2)(gd.numel(), ud.numel()), (ctypes.c_int64 * 2)(inter, inter), None,
+             (ctypes.c_void_p * 2)(g2.data_ptr(), u2.data_ptr()), _stream(torch))
+    okq.call("okq_linear_out_by_in_q", gb.data_ptr(), rows, inter, td, dd.data_ptr(), dd.numel(), hidden, None,
+             out2.data_ptr(), _stream(torch))
+    torch.cuda.synchronize()
+    same = lambda a, b: ((a.view(np.uint32) == b.view(np.uint32)) | (np.isnan(a) & np.isnan(b))).all()
+    h, g, u = gb.cpu().numpy(), g2.cpu().numpy(), u2.cpu().numpy()
+    assert same(ub.cpu().numpy(), u) and same(out.cpu().numpy(), out2.cpu().numpy())
+    with np.errstate(all="ignore"):
+        want = (g * (np.float32(1.0) / (np.float32(1.0) + np.exp(-g)))) * u
+    fine = np.isfinite(want)
+    assert not fine.reshape(rows, inter)[3].all() and np.delete(fine.reshape(rows, inter), 3, 0).all()
+    assert np.all(np.abs(h[fine] - want[fine]) <= 8 * np.spacing(np.abs(want[fine])))
+    assert same(h[~fine], want[~fine])
+
+
 def test_mlp_gated_silu_q_validates_before_launch(torch, okq, orc):
     hidden, inter = 256, 512
     gq = orc.quantize(O.Q4_K, orc.normal(7500, inter * hidden, 0.02))
