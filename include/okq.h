@@ -249,13 +249,16 @@ okq_status okq_rmsnorm_linear_q_multi(const float *x, int64_t rows, int64_t hidd
  * row_bytes(intermediate)); gate_buf, up_buf [rows, intermediate] caller-owned
  * scratch; out [rows, hidden].  Device buffers, x/gate_buf/up_buf 16-byte
  * aligned.  Decode-sized rows (rows <= 8) run gate+up as one grouped GEMV
- * when they share a format.  A single row computes silu(gate) * up on the way
- * (in the gate+up launch where its rows go in pairs, through a per-stream
- * workspace, else in the down GEMV's prologue) whenever the down weight takes
- * the streaming GEMV (gate_buf then holds gate(x)); otherwise silu(gate(x)) * up(x) is left in gate_buf,
- * as the reference does (when gate and up share one decode-batch launch that
- * splits K, by its reduction, or with its tiles in pairs by itself: no separate pass over the intermediate).  up_buf always holds up(x).  Treat both as scratch.  Zero rows, hidden or
- * intermediate are errors (mlp.rs:151-165). */
+ * when they share a format.  silu(gate(x)) * up(x) is left in gate_buf, as the
+ * reference does: by the gate+up launch where its rows (a single row) or tiles
+ * (decode batches) go in pairs, by the reduction of a decode-batch launch that
+ * splits K, by the down GEMM's pre-pass above 32 rows, else by a pass of its own.
+ * Only a single row whose gate and up do not go in pairs (different formats,
+ * Q6_K, hidden above 4096, or few rows) and whose down weight streams computes it in
+ * the down GEMV's prologue; gate_buf then holds gate(x).  up_buf always holds
+ * up(x).  Treat both as scratch.  A single row whose three weights stream uses
+ * no workspace.  Zero rows, hidden or intermediate are errors
+ * (mlp.rs:151-165). */
 okq_status okq_mlp_gated_silu_q(const float *x, int64_t rows, int64_t hidden, int64_t intermediate,
                                 uint32_t gate_type, const void *gate_w, uint64_t gate_bytes, uint32_t up_type,
                                 const void *up_w, uint64_t up_bytes, uint32_t down_type, const void *down_w,

@@ -559,8 +559,8 @@ constexpr int gemv_max_threads() {
 //
 // kPair (two matrices of equal rows, gate then up; dynamic rows of both in a
 // ring of two): a "row" is row i of both matrices, ring slot 0 holding the
-// gate's and slot 1 the up's, so one wave has both sums and writes, besides
-// them, silu(gate) * up to P.h.  The down projection then reads finished
+// gate's and slot 1 the up's, so one wave has both sums and writes up and, in
+// the gate's place, silu(gate) * up.  The down projection then reads finished
 // activations: as its prologue, the SiLU of all 14336 of them in every
 // workgroup, made a Q6_K down launch 17.4 us where it is 14.1 without, and the
 // pairs cost gate + up 0.4 us.
@@ -714,8 +714,10 @@ __device__ __forceinline__ void gemv_body(const uint8_t *__restrict__ W, uint32_
           tot = T == 1 ? sum : tot + sum;
         }
         if constexpr (kPair) {
-          if (lane == 0) y_of(p)[row] = tot;
-          if (p == 1 && lane == 0) P.h[row] = silu_times(gate_sum, tot);
+          if (p == 1 && lane == 0) {
+            y_of(0)[row] = silu_times(gate_sum, tot);
+            y_of(1)[row] = tot;
+          }
           gate_sum = tot;
         } else {
           if (lane == 0) store(row, r, tot + bv);
@@ -866,9 +868,8 @@ __device__ __forceinline__ void gemv_body(const uint8_t *__restrict__ W, uint32_
       auto sum_of = [&](int j) { return wave_sum(F::compute(S[j], xreg[0], xlo[0], wide_rows & 1u, lane)); };
       auto put = [&](float us) {  // lane 0 alone, as below
         if (lane == 0 && row < end) {
-          M.mat[0].y[row] = gs;
+          M.mat[0].y[row] = silu_times(gs, us);
           M.mat[1].y[row] = us;
-          P.h[row] = silu_times(gs, us);
         }
       };
       for (;;) {
@@ -1084,7 +1085,7 @@ template <class F, int D, int XV, bool kMulti, int kPro, int R>
 void launch_kernel(dim3 grid, dim3 block, size_t lds, hipStream_t s, const GemvLaunch &L, const float *x, int k,
                    int T, int G) {
   if constexpr (XV <= 2 && D == 2 && kMulti && kPro == kProNone && R == 1) {
-    if (L.P.h) {
+    if (L.P.pairs) {
       launch_timed(gemv_kernel<F, D, XV, kMulti, kPro, R, true, true>, grid, block, (unsigned)lds, s, L.w, L.bytes, x,
                    L.bias, L.y, L.rows, k, T, G, L.M, L.P, L.nrows);
       return;
@@ -1231,7 +1232,7 @@ hipError_t launch_gemv_multi(int type, const float *x, int64_t K, int64_t rows, 
   if (type != kQ4_K && type != kQ5_K && type != kQ6_K && type != kQ8_0) return hipErrorInvalidValue;
   if (count < 1 || count > kGemvMaxProblems) return hipErrorInvalidValue;
   if (pro.kind != kProNone && rows != 1) return hipErrorNotSupported;  // prologues run one row at a time
-  if (pro.h && (pro.kind != kProNone || rows != 1 || count != 2 || N[0] != N[1] || bias[0] || bias[1] ||
+  if (pro.pairs && (pro.kind != kProNone || rows != 1 || count != 2 || N[0] != N[1] || bias[0] || bias[1] ||
                 !gemv_pairs(type, K, w[0], w[1], N[0], cu_count)))
     return hipErrorInvalidValue;
   GemvLaunch P{};
@@ -1278,7 +1279,7 @@ hipError_t launch_gemv_multi(int type, const float *x, int64_t K, int64_t rows, 
       P.M.start[i - 1] = INT32_MAX;
     }
   }
-  P.rows = (int)(pro.h ? N[0] : total);  // pairs: row i of both matrices
+  P.rows = (int)(pro.pairs ? N[0] : total);  // pairs: row i of both matrices
   if (total == 0) return hipSuccess;
   // up to kMaxRowsPerLaunch activation rows per pass over the weights, as
   // many as the LDS holds: R rows of XRecs plus the teams' partial sums

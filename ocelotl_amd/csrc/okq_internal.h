@@ -57,13 +57,13 @@ constexpr int kGemvMaxProblems = 4;
 // `a` and epsilon `eps`, or the gated SiLU silu(x) * a (x = gate, a = up).
 // A transform needs every matrix of the launch to pass gemv_streams.
 enum GemvProKind { kProNone = 0, kProRms = 1, kProSwiGLU = 2 };
-// `h` (two matrices that gemv_pairs accepts, gate then up, no bias, no
-// prologue): the launch also writes silu(gate) * up [N] there.
+// `pairs` (two matrices that gemv_pairs accepts, gate then up, no bias, no
+// prologue): y[0] receives silu(gate) * up instead of gate.
 struct GemvPro {
   int kind;
   const float *a;
   float eps;
-  float *h;
+  bool pairs;
 };
 bool gemv_streams(int type, int64_t K, const void *w, int64_t N);
 bool gemv_pairs(int type, int64_t K, const void *gate, const void *up, int64_t N, int cu_count);

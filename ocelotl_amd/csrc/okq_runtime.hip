@@ -904,7 +904,7 @@ okq_status okq_rmsnorm_linear_q_multi(const float *x, int64_t rows, int64_t hidd
   const float *nobias[okq::kGemvMaxProblems] = {nullptr, nullptr, nullptr, nullptr};
   const float *const *b = bias ? bias : nobias;
   if (rows == 1 && streams) {  // one decode row: every workgroup normalises x in its prologue
-    const okq::GemvPro pro{okq::kProRms, norm_weight, epsilon, nullptr};
+    const okq::GemvPro pro{okq::kProRms, norm_weight, epsilon, false};
     for (int64_t r = 0; r < rows; ++r) {
       float *o[okq::kGemvMaxProblems];
       for (int i = 0; i < count; ++i) o[i] = out[i] + r * out_features[i];
@@ -985,23 +985,19 @@ okq_status okq_mlp_gated_silu_q(const float *x, int64_t rows, int64_t hidden, in
   // whose split-K reduction then applies the SiLU too)
   bool swiglu_done = false;
   // one row, a down weight that streams: gate and up row by row in pairs, so
-  // that their launch also leaves silu(gate) * up in the neighbours' workspace
-  // and the down GEMV reads it as it is (without that workspace -- a capture
-  // before any such call -- the prologue below computes it)
-  void *hbuf = nullptr;
+  // that their launch leaves silu(gate) * up in gate_buf, as every batch does,
+  // and the down GEMV reads it as it is: one row takes no shared memory
   if (rows == 1 && gate_type == up_type && okq::gemv_streams((int)down_type, intermediate, down_w, hidden) &&
-      okq::gemv_pairs((int)gate_type, hidden, gate_w, up_w, intermediate, info.cu_count) &&
-      get_workspace(dev, s, (size_t)intermediate * sizeof(float), &hbuf, 1) == OKQ_OK) {
+      okq::gemv_pairs((int)gate_type, hidden, gate_w, up_w, intermediate, info.cu_count)) {
     const void *const gw[2] = {gate_w, up_w};
     const int64_t ns[2] = {intermediate, intermediate}, nd = hidden;
     const float *const nob[2] = {nullptr, nullptr};
     float *const os[2] = {gate_buf, up_buf};
-    float *const h = static_cast<float *>(hbuf);
     hipError_t e = okq::launch_gemv_multi((int)gate_type, x, hidden, 1, 2, gw, ns, nob, os, info.cu_count, s,
-                                          okq::GemvPro{okq::kProNone, nullptr, 0.0f, h});
+                                          okq::GemvPro{okq::kProNone, nullptr, 0.0f, true});
     if (e == hipSuccess)
-      e = okq::launch_gemv_multi((int)down_type, h, intermediate, 1, 1, &down_w, &nd, nob, &out, info.cu_count, s,
-                                 okq::GemvPro{});
+      e = okq::launch_gemv_multi((int)down_type, gate_buf, intermediate, 1, 1, &down_w, &nd, nob, &out, info.cu_count,
+                                 s, okq::GemvPro{});
     return hip_status(e, "mlp launch");
   }
   if (gate_type == up_type) {
@@ -1025,7 +1021,7 @@ okq_status okq_mlp_gated_silu_q(const float *x, int64_t rows, int64_t hidden, in
   // gate_buf (the reference's final content of gate_buf) for the other paths:
   // by gate/up's split-K reduction, else by its own pass
   if (rows == 1 && okq::gemv_streams((int)down_type, intermediate, down_w, hidden)) {
-    const okq::GemvPro base{okq::kProSwiGLU, nullptr, 0.0f, nullptr};
+    const okq::GemvPro base{okq::kProSwiGLU, nullptr, 0.0f, false};
     const float *nob = nullptr;
     for (int64_t r = 0; r < rows; ++r) {
       okq::GemvPro pro = base;
