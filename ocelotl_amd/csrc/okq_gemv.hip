@@ -714,11 +714,12 @@ __device__ __forceinline__ void gemv_body(const uint8_t *__restrict__ W, uint32_
           tot = T == 1 ? sum : tot + sum;
         }
         if constexpr (kPair) {
+          const float s = tot + 0.0f;  // as store() writes it: a sum of -0 is +0
           if (p == 1 && lane == 0) {
-            y_of(0)[row] = silu_times(gate_sum, tot);
-            y_of(1)[row] = tot;
+            y_of(0)[row] = silu_times(gate_sum, s);
+            y_of(1)[row] = s;
           }
-          gate_sum = tot;
+          gate_sum = s;
         } else {
           if (lane == 0) store(row, r, tot + bv);
         }
@@ -865,7 +866,9 @@ __device__ __forceinline__ void gemv_body(const uint8_t *__restrict__ W, uint32_
       // next pair's as soon as it is consumed, the pair taken at slot 0
       int row = row_of(0);
       float gs = 0.0f;
-      auto sum_of = [&](int j) { return wave_sum(F::compute(S[j], xreg[0], xlo[0], wide_rows & 1u, lane)); };
+      auto sum_of = [&](int j) {  // as store() writes it: a sum of -0 is +0
+        return wave_sum(F::compute(S[j], xreg[0], xlo[0], wide_rows & 1u, lane)) + 0.0f;
+      };
       auto put = [&](float us) {  // lane 0 alone, as below
         if (lane == 0 && row < end) {
           M.mat[0].y[row] = silu_times(gs, us);

@@ -482,3 +482,27 @@ def test_mlp_one_row_in_pairs_matches_the_grouped_calls(torch, okq, orc, tgu, td
         assert _same_bits(gb3.cpu(), h).all() and _same_bits(ub3.cpu(), u).all()
         assert _same_bits(out3.cpu(), first).all()
     assert np.isnan(first).all() if special == "inf" else np.isfinite(first).all()
+
+
+@pytest.mark.parametrize("t,rows,hidden,inter", [
+    (O.Q8_0, 1, 4096, 8448),   # the GEMV in pairs
+    (O.Q8_0, 8, 1024, 4352),   # decode-batch tiles in pairs
+])
+def test_mlp_in_pairs_stores_sums_of_minus_zero_as_the_grouped_calls(torch, okq, orc, t, rows, hidden, inter):
+    """Zero activations against negative scales sum to -0, which every linear
+    stores as +0 (the bias term of none): gate_buf and up_buf hold +0 too."""
+    print(f"[gpu] mlp pairs, zero sums type={t} rows={rows} hidden={hidden} inter={inter}", flush=True)
+    w = orc.quantize(t, orc.normal(7701, inter * hidden, 0.02)).reshape(-1, O.BLOCK_BYTES[t])
+    w[:, 1] |= 0x80
+    wd, dd = _dev(torch, w.reshape(-1)), _dev(torch, orc.quantize(t, orc.normal(7702, hidden * inter, 0.02)))
+    xd = torch.zeros(rows * hidden, device="cuda")
+    gb, ub, g2, u2 = (torch.full((rows * inter,), 7.0, device="cuda") for _ in range(4))
+    out = torch.full((rows * hidden,), 7.0, device="cuda")
+    okq.call("okq_mlp_gated_silu_q", xd.data_ptr(), rows, hidden, inter, t, wd.data_ptr(), w.size, t, wd.data_ptr(),
+             w.size, t, dd.data_ptr(), dd.numel(), gb.data_ptr(), ub.data_ptr(), out.data_ptr(), _stream(torch))
+    okq.call("okq_gemv_multi", xd.data_ptr(), rows, hidden, t, 2, (ctypes.c_void_p * 2)(wd.data_ptr(), wd.data_ptr()),
+             (ctypes.c_uint64 * 2)(w.size, w.size), (ctypes.c_int64 * 2)(inter, inter), None,
+             (ctypes.c_void_p * 2)(g2.data_ptr(), u2.data_ptr()), _stream(torch))
+    torch.cuda.synchronize()
+    for a in (ub, u2, gb):
+        assert (a.cpu().numpy().view(np.uint32) == 0).all()
