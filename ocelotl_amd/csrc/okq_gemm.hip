@@ -1152,7 +1152,8 @@ __device__ __forceinline__ void dec_run(const void *__restrict__ X, const DecMat
     const int tile = gtile(ltile(ti)), m = mat_of(tile);
     const DecMat &mt = mats.mat[m];
     const int nm = mt.n, col = (tile - mt.tile0) * 16 + cn;
-    const float bv = ksplit == 1 ? Bs[(ti < kDecMaxTiles ? ti : 0) * 256 + wave * 16 + cn] : 0.0f;
+    // (pairs, without a bias: what the SiLU gave as it is, a product of -0 too)
+    const float bv = kPair ? -0.0f : ksplit == 1 ? Bs[(ti < kDecMaxTiles ? ti : 0) * 256 + wave * 16 + cn] : 0.0f;
     // unsplit: the matrix's own output; split: the concatenated partials
     const uint32_t out_end = ksplit > 1 ? part_end : (uint32_t)((size_t)M * nm * 4);
     const Rsrc rs_out = ksplit > 1 ? rs_part : make_rsrc(mt.y, out_end);
@@ -1276,6 +1277,9 @@ __device__ __forceinline__ void dec_run(const void *__restrict__ X, const DecMat
     // the up slot's sums go through its first wave's own place in Red, which
     // no other wave has read, to the gate slot's first wave, kw waves before
     if (writes && bad != 0u) ieee_fix(0, bad);
+    if (writes)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) acc[0][v] += 0.0f;  // as the other launches store it: a sum of -0 is +0
     if (writes && (ts & 1)) Red[wave * 64 + lane] = acc[0];
     __syncthreads();
     if (!writes) return;
@@ -1283,9 +1287,8 @@ __device__ __forceinline__ void dec_run(const void *__restrict__ X, const DecMat
       const f4 up = Red[(wave + kw) * 64 + lane];
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const float gv = acc[0][v] + 0.0f, uv = up[v] + 0.0f;  // as stored: a sum of -0 is +0
-        const float sig = 1.0f / (1.0f + expf(-gv));
-        acc[0][v] = (gv * sig) * uv;
+        const float sig = 1.0f / (1.0f + expf(-acc[0][v]));
+        acc[0][v] = (acc[0][v] * sig) * up[v];
       }
     }
     store(0, acc);

@@ -506,3 +506,28 @@ def test_mlp_in_pairs_stores_sums_of_minus_zero_as_the_grouped_calls(torch, okq,
     torch.cuda.synchronize()
     for a in (ub, u2, gb):
         assert (a.cpu().numpy().view(np.uint32) == 0).all()
+
+
+@pytest.mark.parametrize("t,rows,hidden,inter", [
+    (O.Q8_0, 1, 4096, 8448),    # the GEMV in pairs
+    (O.Q8_0, 8, 1024, 4352),    # decode-batch tiles in pairs
+    (O.Q4_K, 12, 1024, 8448),
+    (O.Q4_K, 24, 1024, 256),    # the split-K reduction
+    (O.Q4_K, 40, 1024, 512),    # the prefill pre-pass
+])
+def test_mlp_keeps_the_sign_of_zero_products(torch, okq, orc, t, rows, hidden, inter):
+    """A gate of zeros times up: silu(0) * up is a zero with up's sign in
+    gate_buf, whichever launch forms it."""
+    print(f"[gpu] mlp zero gate type={t} rows={rows} hidden={hidden} inter={inter}", flush=True)
+    gd = torch.zeros(inter * hidden // O.BLOCK_ELEMS[t] * O.BLOCK_BYTES[t], dtype=torch.uint8, device="cuda")
+    ud, dd, xd = (_dev(torch, a) for a in (orc.quantize(t, orc.normal(7711, inter * hidden, 0.02)),
+                                           orc.quantize(t, orc.normal(7712, hidden * inter, 0.02)),
+                                           orc.normal(7713, rows * hidden, 1.0)))
+    gb, ub = (torch.full((rows * inter,), 7.0, device="cuda") for _ in range(2))
+    out = torch.full((rows * hidden,), 7.0, device="cuda")
+    okq.call("okq_mlp_gated_silu_q", xd.data_ptr(), rows, hidden, inter, t, gd.data_ptr(), gd.numel(), t, ud.data_ptr(),
+             ud.numel(), t, dd.data_ptr(), dd.numel(), gb.data_ptr(), ub.data_ptr(), out.data_ptr(), _stream(torch))
+    torch.cuda.synchronize()
+    h, u = gb.cpu().numpy(), ub.cpu().numpy()
+    assert (h == 0).all() and (np.signbit(h) == np.signbit(u)).all() and 0.4 < np.signbit(h).mean() < 0.6
+    assert (out.cpu().numpy() == 0).all()
