@@ -1311,21 +1311,52 @@ bool gemv_pairs(int type, int64_t K, const void *gate, const void *up, int64_t N
          N < (int64_t)INT32_MAX / 2 && fast_ok(type, K, gate, N) && fast_ok(type, K, up, N);
 }
 
-bool gemv_mixes(int64_t K, int count, const int *types, const void *const *w, const int64_t *N) {
-  int64_t n4 = 0, n6 = 0;
+// A mixed launch's workgroups by weight bytes, one per CU (cu_count >= 2): of
+// each format (Q4_K, Q6_K), and the rows that its waves (or teams of T waves)
+// stream one after the other at the largest team count.
+namespace {
+struct MixedShare {
+  int64_t nb[2], steps[2];
+};
+MixedShare mixed_share(int64_t K, const int64_t rows[2], int cu_count) {
+  const int64_t T = (K / 64 + 63) / 64, max_g = std::max<int64_t>(1, 16 / T);
+  const int64_t b4 = rows[0] * (int64_t)row_bytes_of(kQ4_K, K), all = b4 + rows[1] * (int64_t)row_bytes_of(kQ6_K, K);
+  MixedShare m;
+  m.nb[0] = std::min<int64_t>(std::max<int64_t>(1, (cu_count * b4 + all / 2) / all), cu_count - 1);
+  m.nb[1] = cu_count - m.nb[0];
+  for (int f = 0; f < 2; ++f) m.steps[f] = (rows[f] + m.nb[f] * max_g - 1) / (m.nb[f] * max_g);
+  return m;
+}
+}  // namespace
+
+// Every matrix streams, and in few steps: the mixed kernel has the one-row
+// ring and a fixed row order, which over many steps lose to the separate
+// launches' deeper ring and rows handed out as waves get free (one wave per
+// row), by more than the launch saved (~2.4 us).  That shows early where many
+// lanes of a row's waves idle, later where K fills them.  Two launches over
+// one, by the larger step count (us):
+//   K 4096: 2 steps 10.1 / 7.6, 5 13.8 / 12.5, 8 20.2 / 18.4, 13 26.9 / 24.9, 64 (the head) 82.6 / 108.0
+//   K 1024 to 3072: 3 steps 9.4 / 7.9, 6 11.0 to 15.1 / 11.2 to 14.4, 7 11.7 to 14.3 / 13.1 to 14.6, 10 14.1 / 16.5
+//   K 5120 (teams of two waves, 80 of 128 lanes): 7 steps 16.7 / 13.8, 9 17.2 / 18.2, 17 27.1 / 30.8
+//   K 8192: 6 steps 16.8 / 13.8, 33 62.7 / 60.2; K 14336: 7 19.6 / 16.3, 34 60.5 / 57.8, 52 80.9 / 86.1
+bool gemv_mixes(int64_t K, int count, const int *types, const void *const *w, const int64_t *N, int cu_count) {
+  int64_t n[2] = {0, 0};
   for (int i = 0; i < count; ++i) {
     if (N[i] < 1 || (types[i] != kQ4_K && types[i] != kQ6_K) || !fast_ok(types[i], K, w[i], N[i])) return false;
-    (types[i] == kQ4_K ? n4 : n6) += N[i];
+    n[types[i] == kQ4_K ? 0 : 1] += N[i];
   }
-  return n4 > 0 && n6 > 0 && n4 < (int64_t)INT32_MAX && n6 < (int64_t)INT32_MAX;
+  if (cu_count < 2 || n[0] < 1 || n[1] < 1 || n[0] >= (int64_t)INT32_MAX || n[1] >= (int64_t)INT32_MAX) return false;
+  const MixedShare m = mixed_share(K, n, cu_count);
+  const int64_t most = K < 4096 ? 6 : K == 4096 ? 13 : K / 64 * 8 >= (K + 4095) / 4096 * 64 * 7 ? 32 : 8;
+  return std::max(m.steps[0], m.steps[1]) <= most;
 }
 
 hipError_t launch_gemv_mixed(const float *x, int64_t K, int count, const int *types, const void *const *w,
                              const int64_t *N, const float *const *bias, float *const *y, int cu_count,
                              hipStream_t s) {
-  if (!gemv_mixes(K, count, types, w, N) || cu_count < 2) return hipErrorInvalidValue;
+  if (!gemv_mixes(K, count, types, w, N, cu_count)) return hipErrorInvalidValue;
   GemvMore M[2] = {};
-  int64_t rows[2] = {0, 0}, bytes[2] = {0, 0};
+  int64_t rows[2] = {0, 0};
   for (int f = 0; f < 2; ++f) {
     const int t = f == 0 ? kQ4_K : kQ6_K;
     int c = 0;
@@ -1335,7 +1366,6 @@ hipError_t launch_gemv_mixed(const float *x, int64_t K, int count, const int *ty
       M[f].mat[c] = GemvMat{static_cast<const uint8_t *>(w[i]), bias[i], y[i], (uint32_t)b, (int)rows[f], (int)N[i], 0};
       if (c > 0) M[f].start[c - 1] = (int)rows[f];
       rows[f] += N[i];
-      bytes[f] += (int64_t)b;
       ++c;
     }
     for (; c < kGemvMaxProblems; ++c) {
@@ -1343,16 +1373,14 @@ hipError_t launch_gemv_mixed(const float *x, int64_t K, int count, const int *ty
       if (c > 0) M[f].start[c - 1] = INT32_MAX;
     }
   }
-  // workgroups by bytes; per format the fewest teams that finish in as many
-  // steps as the most would (launch_stream's rule)
+  // per format the fewest teams that finish in as many steps as the most
+  // would (launch_stream's rule)
   const int U = (int)(K / 64), T = (U + 63) / 64;
   const int64_t max_g = std::max(1, 16 / T);
-  int64_t nb[2], G[2];
-  nb[0] = std::min<int64_t>(std::max<int64_t>(1, (cu_count * bytes[0] + (bytes[0] + bytes[1]) / 2) / (bytes[0] + bytes[1])),
-                            cu_count - 1);
-  nb[1] = cu_count - nb[0];
+  const MixedShare share = mixed_share(K, rows, cu_count);
+  int64_t nb[2] = {share.nb[0], share.nb[1]}, G[2];
   for (int f = 0; f < 2; ++f) {
-    const int64_t steps = (rows[f] + nb[f] * max_g - 1) / (nb[f] * max_g);
+    const int64_t steps = share.steps[f];
     G[f] = std::min<int64_t>(max_g, (rows[f] + nb[f] * steps - 1) / (nb[f] * steps));
     nb[f] = std::min<int64_t>(nb[f], (rows[f] + G[f] * steps - 1) / (G[f] * steps));
   }

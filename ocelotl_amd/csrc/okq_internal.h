@@ -69,8 +69,8 @@ bool gemv_streams(int type, int64_t K, const void *w, int64_t N);
 bool gemv_pairs(int type, int64_t K, const void *gate, const void *up, int64_t N, int cu_count);
 // Q4_K and Q6_K matrices (at least one of each, types[i] per matrix) against
 // one activation row in one launch; each result is its own launch's bit for
-// bit.  gemv_mixes: every matrix streams.
-bool gemv_mixes(int64_t K, int count, const int *types, const void *const *w, const int64_t *N);
+// bit.  gemv_mixes: every matrix streams, in few enough steps to pay.
+bool gemv_mixes(int64_t K, int count, const int *types, const void *const *w, const int64_t *N, int cu_count);
 hipError_t launch_gemv_mixed(const float *x, int64_t K, int count, const int *types, const void *const *w,
                              const int64_t *N, const float *const *bias, float *const *y, int cu_count, hipStream_t s);
 // x [rows, K] and y[i] [rows, N[i]] row-major; every pass over the weights

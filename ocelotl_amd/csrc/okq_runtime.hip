@@ -783,7 +783,7 @@ okq_status okq_linear_multi_q(const float *x, int64_t rows, int64_t in_features,
       mb[c] = b[i];
       mo[c++] = out[i];
     }
-    if (c > 1 && okq::gemv_mixes(in_features, c, types, mw, mn)) {
+    if (c > 1 && okq::gemv_mixes(in_features, c, types, mw, mn, info.cu_count)) {
       st = hip_status(okq::launch_gemv_mixed(x, in_features, c, types, mw, mn, mb, mo, info.cu_count, s),
                       "linear_multi launch");
       if (st != OKQ_OK) return st;
