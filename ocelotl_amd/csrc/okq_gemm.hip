@@ -1596,22 +1596,37 @@ bool gemm_supported(int type, int64_t M, int64_t K, int64_t N) {
 
 static size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
 
+// Bytes of a plan's split-K partials; the slices that f32_split may choose at
+// most, and the bytes of their partials in calls whose planes exceed
+// kScratchBytes (others: what the planes leave of it).  Both bounds together
+// keep a larger call's reserve above every smaller call's need.  The second
+// cuts few splits, those of large outputs, where the partials' own traffic has
+// eaten most of the gain: Q6_K, K 28672 -> 8192, us per call without it / with
+// it: 1143 rows 1454 / 1480 (7 slices, 5), 2200 2809 / 2936 (4, 2), 3500 4289 /
+// 4631 (2, 1); K 14080 -> 4731 at 1805 rows (bf16) uncut.  At 128 MiB: 3160 at 2200.
+static size_t part_bytes(int64_t ks, int64_t M, int64_t N) {
+  return ks > 1 ? up256((size_t)ks * (size_t)M * (size_t)N * sizeof(float)) : 0;
+}
+constexpr int64_t kMostSlices = 16;
+constexpr size_t kMostPartBytes = 192u << 20;
+
 // K slices of gemm_f32_kernel for one matrix: the split of least estimated
 // time.  A round of workgroups (one per CU) takes ~7 us (Q4_K, both planes;
 // one plane: the MFMAs of one) per super-block of its slice and ~5 us around
 // its loop; the partials are written and read once at ~4 TB/s, and their
 // reduction is one more launch.
-static int64_t f32_split(int type, int64_t M, int64_t N, int64_t K, bool one_plane, int cu_count) {
+static int64_t f32_split(int type, int64_t M, int64_t N, int64_t K, bool one_plane, size_t part_limit, int cu_count) {
   const double us_sb = (type == kQ6_K ? 10.0 : type == kQ8_0 ? 8.5 : 7.0) * (one_plane ? 0.7 : 1.0) *
                        (0.2 + 0.2 * gemm_f32_blocks(M));
   const int64_t nsb = K / 256, tiles = gemm_f32_tiles(M, N), cus = cu_count;
   int64_t best = 1;
   double least = 0.0;
   // (Q6_K in slices of one super-block: 1.80e-7 from float64, of two 1.73e-7)
-  const int64_t most = std::min<int64_t>(16, type == kQ6_K ? std::max<int64_t>(1, nsb / 2) : nsb);
+  const int64_t most = std::min<int64_t>(kMostSlices, type == kQ6_K ? std::max<int64_t>(1, nsb / 2) : nsb);
   for (int64_t ks = 1; ks <= most; ++ks) {
     const double bytes = 4.0 * (double)M * (double)N * (double)(2 * ks + 1);
-    if (ks > 1 && bytes > (double)UINT32_MAX) break;  // the reduction's 32-bit offsets, with room
+    // the reduction's 32-bit offsets, with room, and the partials' own bound
+    if (ks > 1 && (bytes > (double)UINT32_MAX || part_bytes(ks, M, N) > part_limit)) break;
     const double us = (double)((tiles * ks + cus - 1) / cus) * (us_sb * (double)((nsb + ks - 1) / ks) + 5.0) +
                       (ks > 1 ? 3.0 + bytes / 4e6 : 0.0);
     if (ks == 1 || us < least) best = ks, least = us;
@@ -1628,6 +1643,10 @@ GemmPlan gemm_plan(int type, int64_t M, int64_t N, int64_t K, bool x_is_bf16, in
   // (Q6_K grids that fill its tiles), okq_gemm_f32.hip with one plane otherwise.
   const int64_t nsb = K / 256;
   int64_t ks = 1;
+  // the pre-pass's planes, sums and row scales
+  const size_t plane = (size_t)M * (size_t)K * sizeof(_Float16);
+  const size_t sums = (size_t)M * (size_t)(K / 32) * 2 * sizeof(_Float16);
+  const size_t off_part = up256(plane) * (x_is_bf16 ? 1 : 2) + up256(sums) + up256((size_t)M * sizeof(float));
   if (M <= kDecRows) {
     // decode batch: the streaming kernel.  K slices small enough for the
     // activations to fit the LDS budget (M rows of 1 or 2 planes of the slice plus
@@ -1655,9 +1674,7 @@ GemmPlan gemm_plan(int type, int64_t M, int64_t N, int64_t K, bool x_is_bf16, in
       p.kwaves = (int)(kDecWaves / T);
       p.groups = (int)((ntiles + T - 1) / T);
       p.ksplit = 1;
-      p.off_lo = p.off_sums = p.off_rscale = p.off_part = 0;
-      p.workspace = 0;
-      return p;
+      return p;  // no workspace
     }
     // one workgroup (16 waves) per CU: column groups of 16 tiles, at most one
     // per CU (waves then take several tiles), and as many K slices as fit in
@@ -1696,7 +1713,7 @@ GemmPlan gemm_plan(int type, int64_t M, int64_t N, int64_t K, bool x_is_bf16, in
     if (!x_is_bf16) {
       p.bm = 128;
       p.wide = 5;
-      ks = f32_split(type, M, N, K, false, cu_count);
+      ks = f32_split(type, M, N, K, false, off_part > kScratchBytes ? kMostPartBytes : SIZE_MAX, cu_count);
     } else if (type == kQ8_0) {
       // gemm_q8_kernel (bf16 activations straight from x: no pre-pass).  The
       // 8-wave 128 x 256 tiles (one workgroup per CU) while they fill at
@@ -1723,7 +1740,7 @@ GemmPlan gemm_plan(int type, int64_t M, int64_t N, int64_t K, bool x_is_bf16, in
     } else if (!reg_dequant) {
       p.bm = 128;
       p.wide = 6;
-      ks = f32_split(type, M, N, K, true, cu_count);
+      ks = f32_split(type, M, N, K, true, kMostPartBytes, cu_count);
     } else {
       p.bm = 128;
       const int64_t cus = cu_count;
@@ -1750,30 +1767,33 @@ GemmPlan gemm_plan(int type, int64_t M, int64_t N, int64_t K, bool x_is_bf16, in
     }
   }
   p.ksplit = (int)std::max<int64_t>(1, ks);
-  auto up = up256;
-  if (p.bm == kDecRows) {  // the decode-batch kernel needs only the split-K partials (whole 16-column tiles)
-    p.off_lo = p.off_sums = p.off_rscale = p.off_part = 0;
-    p.workspace = p.ksplit > 1 ? up((size_t)p.ksplit * M * ((N + 15) / 16 * 16) * sizeof(float)) : 0;
+  if (p.bm == kDecRows || p.wide == 3) {
+    // only the split-K partials: the decode-batch kernel converts x itself
+    // (whole 16-column tiles), the Q8_0 bf16 kernel reads it as it is
+    p.reserve = p.workspace = part_bytes(p.ksplit, M, p.wide == 3 ? N : (N + 15) / 16 * 16);
     return p;
   }
-  if (p.wide == 3) {  // the Q8_0 bf16 kernel reads x itself: only the split-K partials
-    p.off_lo = p.off_sums = p.off_rscale = p.off_part = 0;
-    p.workspace = p.ksplit > 1 ? up((size_t)p.ksplit * M * N * sizeof(float)) : 0;
-    return p;
-  }
-  const size_t plane = (size_t)M * (size_t)K * sizeof(_Float16);
-  const size_t sums = (size_t)M * (size_t)(K / 32) * 2 * sizeof(_Float16);
-  p.off_lo = up(plane);
-  p.off_sums = p.off_lo + (x_is_bf16 ? 0 : up(plane));
-  p.off_rscale = p.off_sums + up(sums);
-  p.off_part = p.off_rscale + up((size_t)M * sizeof(float));
-  auto parts = [&](int k) { return k > 1 ? up((size_t)k * M * N * sizeof(float)) : (size_t)0; };
+  p.off_lo = up256(plane);
+  p.off_sums = p.off_lo + (x_is_bf16 ? 0 : up256(plane));
+  p.off_rscale = p.off_sums + up256(sums);
+  p.off_part = off_part;
   // a call whose planes fit the allocation-free entry point's scratch stays
   // within it (one dispatch for both entry points: the same bits)
   if (p.wide == 5 && p.off_part <= kScratchBytes)
-    while (p.ksplit > 1 && p.off_part + parts(p.ksplit) > kScratchBytes) --p.ksplit;
-  p.workspace = p.off_part + parts(p.ksplit);
+    while (p.ksplit > 1 && p.off_part + part_bytes(p.ksplit, M, N) > kScratchBytes) --p.ksplit;
+  p.reserve = p.workspace = p.off_part + part_bytes(p.ksplit, M, N);
+  if (!x_is_bf16 || type == kQ6_K) {  // calls that f32_split splits, or would at fewer rows
+    const size_t limit = x_is_bf16 || p.off_part > kScratchBytes ? kMostPartBytes : kScratchBytes - p.off_part;
+    p.reserve = std::max(p.reserve, p.off_part + std::min(limit, part_bytes(std::min(kMostSlices, nsb), M, N)));
+  }
   return p;
+}
+
+bool gemm_plan_lower(GemmPlan &p, int64_t M, int64_t N) {
+  if (p.wide < 5 || p.ksplit <= 1) return false;
+  --p.ksplit;
+  p.workspace = p.off_part + part_bytes(p.ksplit, M, N);
+  return true;
 }
 
 PrefillPlan prefill_plan(int64_t M, int64_t K, int count, const int *types, const int64_t *N, int cu_count) {
@@ -1783,10 +1803,11 @@ PrefillPlan prefill_plan(int64_t M, int64_t K, int count, const int *types, cons
     g.ksplit[i] = p.ksplit;
     if (i == 0) {
       g.base = p;
-      g.workspace = p.off_part;
+      g.workspace = g.reserve = p.off_part;
     }
     g.off_part[i] = g.workspace;
     g.workspace += p.workspace - p.off_part;
+    g.reserve += p.reserve - p.off_part;
   }
   return g;
 }

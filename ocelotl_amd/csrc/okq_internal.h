@@ -103,10 +103,18 @@ struct GemmPlan {
                        // 5 f32 activations, every format, 6 bf16 ones in its one-plane form
                        // (32 gemm_f32_blocks(M) x 256 tiles)
   size_t off_lo, off_sums, off_rscale, off_part, workspace;
+  // what a stream's workspace grows to for this call (>= workspace): at least
+  // what any call with no more rows, inputs and outputs needs (gemm_f32_kernel's
+  // K split, and with it the partials, rises and falls with the rows; every
+  // other plan: the call's own need)
+  size_t reserve;
 };
 // Size of the allocation-free entry point's static scratch.
 constexpr size_t kScratchBytes = 64u << 20;
 GemmPlan gemm_plan(int type, int64_t M, int64_t N, int64_t K, bool x_is_bf16, int cu_count);
+// The same plan with one K slice (and its partials) fewer; false when it has
+// one slice or another kernel's.
+bool gemm_plan_lower(GemmPlan &p, int64_t M, int64_t N);
 // `workspace` holds plan.workspace bytes (256-aligned); it is reused by later
 // calls on the stream.
 hipError_t launch_gemm(int type, const void *x, bool x_is_bf16, int64_t M, int64_t K, const void *w, int64_t N,
@@ -192,7 +200,7 @@ int gemm_f32_tiles(int64_t M, int64_t N);
 struct PrefillPlan {
   GemmPlan base;  // the planes' layout
   int ksplit[kPrefillMats];
-  size_t off_part[kPrefillMats], workspace;
+  size_t off_part[kPrefillMats], workspace, reserve;  // as GemmPlan's
 };
 // What the pre-pass forms from x first (kind: GemvProKind): nothing, the
 // RMSNorm of x with weight a (out: scratch [M][K], written for rows holding

@@ -6,7 +6,9 @@
 // error conventions of docs/design/kernels.md:96-99.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdarg>
+#include <cstdint>
 #include <cstdio>
 #include <cstring>
 #include <map>
@@ -201,8 +203,13 @@ okq_status validate_rmsnorm(const float *x, int64_t rows, int64_t hidden, const 
 // One buffer per (device, stream, slot): work on one stream is ordered, so
 // reuse is safe; different streams never share.  Grows on demand; growing is
 // refused while the stream is being captured into a graph (allocation is not
-// capturable), so a caller that captures must run one call of at least the
-// same size on that stream first.
+// capturable), so a caller that captures must run the call on that stream
+// first, or, above 32 rows of f32 activations (and of bf16 ones against Q6_K),
+// one with at least its rows, inputs and outputs: its growth covers the
+// smaller call's plan too (GemmPlan::reserve).  Where no memory is left
+// for that, or a capture finds a buffer for the call's planes but not for all
+// its partials, the K split is lowered until they fit (the last bits of a
+// result follow its split).
 //
 // A buffer is never freed once handed out.  A graph captured earlier keeps
 // the pointer it recorded, and another host thread may have looked up the
@@ -216,6 +223,7 @@ okq_status validate_rmsnorm(const float *x, int64_t rows, int64_t hidden, const 
 struct Workspace {
   void *ptr = nullptr;
   size_t bytes = 0;
+  size_t refused = SIZE_MAX;  // an allocation that failed: asked for again only where a call needs it all
 };
 std::mutex g_ws_mutex;
 std::map<std::tuple<int, hipStream_t, int>, Workspace> g_ws;
@@ -223,29 +231,55 @@ std::map<std::tuple<int, hipStream_t, int>, Workspace> g_ws;
 // Slot 0 serves the linear itself (GEMM planes, bf16 widening); slot 1 holds
 // a neighbour's output (normalised or gated activations) that a linear then
 // reads, so the two never alias.
-okq_status get_workspace(int dev, hipStream_t s, size_t bytes, void **out, int slot = 0) {
+enum class Grow { Ok, Capture, Alloc };
+
+// At least `bytes`; a buffer that has to grow, or could outside a capture,
+// grows to half again of `reserve` (>= bytes), or to `bytes` where that fails.
+Grow grow_workspace(int dev, hipStream_t s, size_t bytes, size_t reserve, void **out, int slot = 0) {
   std::lock_guard<std::mutex> lock(g_ws_mutex);
   Workspace &w = g_ws[{dev, s, slot}];
-  if (w.bytes >= bytes) {
-    *out = w.ptr;
-    return ok();
-  }
+  *out = w.ptr;
+  if (w.bytes >= reserve) return Grow::Ok;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone)
+    return w.bytes >= bytes ? Grow::Ok : Grow::Capture;
+  for (const size_t want : {reserve + reserve / 2, bytes}) {
+    if (want <= w.bytes) return Grow::Ok;
+    if (want > bytes && want >= w.refused) continue;
+    void *p = nullptr;
+    if (hipMalloc(&p, want) == hipSuccess) {
+      w.ptr = p;  // the previous buffer (if any) stays allocated: see above
+      w.bytes = want;
+      *out = p;
+      return Grow::Ok;
+    }
+    (void)hipGetLastError();  // callers go on with a smaller workspace: the next launch check must not see this error
+    w.refused = std::min(w.refused, want);
+  }
+  return Grow::Alloc;
+}
+
+okq_status workspace_status(Grow g, size_t bytes) {
+  if (g == Grow::Capture)
     return fail(OKQ_E_ALLOC,
                 "hip-gfx950: GEMM workspace of %zu bytes is not allocated for this stream and cannot be allocated "
                 "during graph capture; run one call of this size on the stream before capturing",
                 bytes);
-  const size_t want = bytes + bytes / 2;
-  void *p = nullptr;
-  if (hipMalloc(&p, want) != hipSuccess) {
-    (void)hipGetLastError();  // callers go on with a smaller workspace: the next launch check must not see this error
-    return fail(OKQ_E_ALLOC, "hip-gfx950: hipMalloc of a %zu-byte GEMM workspace failed", want);
-  }
-  w.ptr = p;  // the previous buffer (if any) stays allocated: see above
-  w.bytes = want;
-  *out = w.ptr;
+  if (g == Grow::Alloc) return fail(OKQ_E_ALLOC, "hip-gfx950: hipMalloc of a %zu-byte GEMM workspace failed", bytes);
   return ok();
+}
+
+okq_status get_workspace(int dev, hipStream_t s, size_t bytes, void **out, int slot = 0) {
+  return workspace_status(grow_workspace(dev, s, bytes, bytes, out, slot), bytes);
+}
+
+// The workspace of a plan, its K split lowered where it cannot be had.
+okq_status gemm_workspace(int dev, hipStream_t s, okq::GemmPlan &plan, int64_t M, int64_t N, void **out) {
+  Grow g;
+  while ((g = grow_workspace(dev, s, plan.workspace, plan.reserve, out)) != Grow::Ok &&
+         okq::gemm_plan_lower(plan, M, N)) {
+  }
+  return workspace_status(g, plan.workspace);
 }
 
 // Calls that take workspace enqueue several kernels (activation pre-pass,
@@ -360,7 +394,7 @@ okq_status linear_impl(const void *x, bool x_bf16, int64_t rows, int64_t K, uint
   }
   if (use_gemm) {
     void *ws = nullptr;
-    const okq::GemmPlan plan = okq::gemm_plan((int)type, rows, N, K, x_bf16, info.cu_count);
+    okq::GemmPlan plan = okq::gemm_plan((int)type, rows, N, K, x_bf16, info.cu_count);
     if (sc.fixed) {
       if (plan.workspace > kScratchBytes)
         return fail(OKQ_E_SHAPE,
@@ -369,7 +403,7 @@ okq_status linear_impl(const void *x, bool x_bf16, int64_t rows, int64_t K, uint
                     (long long)rows, (long long)K, (long long)N, plan.workspace, kScratchBytes);
       st = scratch_for(dev, &ws);
     } else {
-      st = get_workspace(dev, s, plan.workspace, &ws);
+      st = gemm_workspace(dev, s, plan, rows, N, &ws);
     }
     if (st != OKQ_OK) return st;
     return hip_status(okq::launch_gemm((int)type, x, x_bf16, rows, K, w, N, bias, out, ws, plan, s), "gemm launch");
@@ -585,15 +619,15 @@ okq_status okq_linear_out_by_in_q_bf16(const uint16_t *x, int64_t rows, int64_t 
 // More than 32 f32 rows through `count` MFMA-routed matrices (the stream's
 // enqueue lock held): bit for bit each matrix's own call.  Where the shared
 // workspace cannot be had (a capture before any call of this size), the
-// matrices run one by one, each within the workspace of its own call, after
-// `pro` as a pass of its own.
+// matrices run one by one, each within the workspace of its own call (its K
+// split lowered if need be), after `pro` as a pass of its own.
 static okq_status prefill_multi(const float *x, int64_t rows, int64_t K, int count, const int *types,
                                 const void *const *w, const int64_t *N, const float *const *bias, float *const *out,
                                 hipStream_t s, int dev, const DevInfo &info,
                                 const okq::PrepPro &pro = okq::PrepPro{}) {
   const okq::PrefillPlan plan = okq::prefill_plan(rows, K, count, types, N, info.cu_count);
   void *ws = nullptr;
-  if (get_workspace(dev, s, plan.workspace, &ws) == OKQ_OK)
+  if (grow_workspace(dev, s, plan.workspace, plan.reserve, &ws) == Grow::Ok)
     return hip_status(okq::launch_prefill_multi(x, rows, K, count, types, w, N, bias, out, ws, plan, s, pro),
                       "grouped gemm launch");
   if (pro.kind != okq::kProNone) {
@@ -603,8 +637,8 @@ static okq_status prefill_multi(const float *x, int64_t rows, int64_t K, int cou
     x = pro.out;
   }
   for (int i = 0; i < count; ++i) {
-    const okq::GemmPlan p = okq::gemm_plan(types[i], rows, N[i], K, false, info.cu_count);
-    okq_status st = get_workspace(dev, s, p.workspace, &ws);
+    okq::GemmPlan p = okq::gemm_plan(types[i], rows, N[i], K, false, info.cu_count);
+    okq_status st = gemm_workspace(dev, s, p, rows, N[i], &ws);
     if (st != OKQ_OK) return st;
     st = hip_status(okq::launch_gemm(types[i], x, false, rows, K, w[i], N[i], bias[i], out[i], ws, p, s), "gemm launch");
     if (st != OKQ_OK) return st;

@@ -7,6 +7,7 @@ may have looked the buffer up without having enqueued its kernel yet.  So a
 larger call on the same stream moves the stream to a new, larger buffer and
 leaves the old one alone.
 """
+import ctypes
 import threading
 
 import numpy as np
@@ -157,3 +158,87 @@ def test_graph_replayed_on_another_stream_after_its_capture_stream_is_idle(torch
         assert (out.cpu().numpy().view(np.uint32) == ref.cpu().numpy().view(np.uint32)).all(), rep
         assert (bo.cpu().numpy().view(np.uint32) == want_busy.view(np.uint32)).all(), rep
     del g
+
+
+def _random_problem(torch, okq, t, rows, n, k, seed):
+    """A problem with its weights quantised on the device (a reference call's
+    operands, not an oracle's)."""
+    s = torch.cuda.current_stream().cuda_stream
+    w = torch.empty(n * k, dtype=torch.float32, device="cuda")
+    okq.call("okq_fill_normal", seed, 0, n * k, 0.02, w.data_ptr(), s)
+    wq = torch.empty(n * k // O.BLOCK_ELEMS[t] * O.BLOCK_BYTES[t], dtype=torch.uint8, device="cuda")
+    okq.call("okq_quantize", t, w.data_ptr(), n * k, wq.data_ptr(), s)
+    x = torch.empty(rows * k, dtype=torch.float32, device="cuda")
+    okq.call("okq_fill_normal", seed + 1, 0, rows * k, 1.0, x.data_ptr(), s)
+    torch.cuda.synchronize()
+    return wq, x
+
+
+def _own_stream(torch):
+    """A stream that no earlier test has used (torch's come from a pool)."""
+    hip, raw = ctypes.CDLL("libamdhip64.so"), ctypes.c_void_p()
+    assert hip.hipStreamCreate(ctypes.byref(raw)) == 0
+    return torch.cuda.ExternalStream(raw.value)
+
+
+@pytest.mark.parametrize("t", [O.Q6_K, O.Q8_0])
+def test_a_call_of_more_rows_allows_the_capture_of_one_of_fewer(torch, okq, t):
+    """1568 rows run eagerly on a stream; 1135 rows, whose K split needs more
+    partials, are then captured on it and replay to the eager bits."""
+    n, k = 4096, 14336
+    print(f"[gpu] workspace of a larger call type={t}", flush=True)
+    wq, x = _random_problem(torch, okq, t, 1568, n, k, 9300)
+
+    def call(rows, out, stream):
+        okq.call("okq_linear_out_by_in_q", x.data_ptr(), rows, k, t, wq.data_ptr(), wq.numel(), n, None, out.data_ptr(),
+                 stream)
+
+    big, want, out = (torch.full((r * n,), 7.0, device="cuda") for r in (1568, 1135, 1135))
+    call(1135, want, torch.cuda.current_stream().cuda_stream)
+    side = _own_stream(torch)
+    torch.cuda.synchronize()
+    call(1568, big, side.cuda_stream)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        call(1135, out, side.cuda_stream)
+    for _ in range(3):
+        out.fill_(7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int32), want.view(torch.int32))
+        call(1135, want, torch.cuda.current_stream().cuda_stream)
+
+
+def test_a_capture_takes_the_split_that_the_held_workspace_allows(torch, okq):
+    """A stream that has served a few outputs holds the planes of 128 rows, not
+    the partials of 14336 outputs: the capture takes fewer K slices, the same
+    values but for the order of their sums (each sum of exact products in
+    f32: 2e-6 of the result's norm), and leaves no error behind."""
+    t, rows, n, k = O.Q4_K, 128, 14336, 4096
+    print("[gpu] split lowered under capture", flush=True)
+    wq, x = _random_problem(torch, okq, t, rows, n, k, 9310)
+
+    def call(cols, out, stream):
+        okq.call("okq_linear_out_by_in_q", x.data_ptr(), rows, k, t, wq.data_ptr(), wq.numel() // n * cols, cols, None,
+                 out.data_ptr(), stream)
+
+    few, want, out = (torch.full((rows * c,), 7.0, device="cuda") for c in (64, n, n))
+    call(n, want, torch.cuda.current_stream().cuda_stream)
+    side = _own_stream(torch)
+    torch.cuda.synchronize()
+    call(64, few, side.cuda_stream)
+    torch.cuda.synchronize()
+    with pytest.raises(okq.OkqStatusError):  # a message that a failure inside the capture would replace
+        okq.call("okq_rmsnorm", x.data_ptr(), 1, 0, x.data_ptr(), 1e-5, x.data_ptr(), side.cuda_stream)
+    before = okq.last_error()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        call(n, out, side.cuda_stream)
+    assert okq.last_error() == before
+    for _ in range(3):
+        out.fill_(7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert not torch.equal(out, want)
+        assert ((out - want).double().norm() <= 2e-6 * want.double().norm()).item()
