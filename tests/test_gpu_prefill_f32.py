@@ -97,6 +97,31 @@ def test_bf16_q6k_prefill_on_small_grids_matches_float64(torch, okq, orc, rows, 
     assert bool((err <= bound).all()), float((err / bound).max())
 
 
+@pytest.mark.parametrize("t", [O.Q4_K, O.Q5_K])
+def test_bf16_prefill_on_weights_near_4_gib_matches_float64(torch, okq, orc, t):
+    """bf16 activations through Q4_K and Q5_K tensors too close to 4 GiB for the
+    kernels that address a padded column tile: the one-plane form, at its three
+    tile heights, the last column tile and rows ragged.  The tensor repeats
+    4093 rows, so that no tile sees the same columns twice; bounds as above."""
+    k, base = 7168, 4093
+    row = k // 256 * O.BLOCK_BYTES[t]
+    n = ((1 << 32) - 1025) // row - 141
+    wq = orc.quantize(t, orc.normal(9400 + t, base * k, 0.02))
+    w = _dev(torch, orc.dequantize(t, wq, base * k)).view(base, k).double()
+    wd = _dev(torch, wq).view(base, row).repeat((n + base - 1) // base, 1)[:n].contiguous().view(-1)
+    for rows in (33, 70, 127):
+        print(f"[gpu] bf16 prefill near 4 GiB type={t} rows={rows} K={k} N={n}", flush=True)
+        x = _dev(torch, orc.normal(9401 + rows, rows * k, 1.0)).view(rows, k).to(torch.bfloat16)
+        out = _linear(torch, okq, t, x, rows, k, wd, n, entry="okq_linear_out_by_in_q_bf16").view(rows, n)
+        torch.cuda.synchronize()
+        want = x.double() @ w.t()
+        bound = 2.0 ** -20 * x.double().abs().sum(1, keepdim=True) * 2 * w.abs().amax(1) + 2.0 ** -22 * want.abs()
+        for c in range(0, n, base):
+            m = min(base, n - c)
+            err = (out[:, c:c + m].double() - want[:, :m]).abs()
+            assert bool((err <= bound[:, :m]).all()), (c, float((err / bound[:, :m]).max()))
+
+
 @pytest.mark.parametrize("types,rows,k,ns", [
     ([O.Q4_K, O.Q4_K, O.Q6_K], 70, 4096, [1024, 256, 256]),
     ([O.Q8_0, O.Q8_0, O.Q8_0], 333, 2048, [2048, 512, 300]),
