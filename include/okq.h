@@ -189,12 +189,12 @@ okq_status okq_gemm_bf16(const uint16_t *x, int64_t rows, int64_t in_features, u
  * matrix is validated like okq_gemv before anything launches.  A matrix that
  * okq_linear_out_by_in_q would not give to the GEMV at this row count (the
  * large weights of its 3-8 row rule, every weight above 8 rows) is computed
- * by the MFMA kernels
- * instead: alone through that entry
- * point's dispatch, or -- two or more of them at up to 32 rows -- together in
- * one decode-batch launch whose K split follows their combined columns.
- * Outputs equal okq_linear_out_by_in_q's on each matrix bit for bit, except
- * those of such a shared decode-batch launch, which agree within the
+ * by the MFMA kernels instead: alone through that entry point's dispatch, or,
+ * two or more of them, together: at up to 32 rows in one decode-batch launch
+ * whose K split follows their combined columns, above 32 rows with one
+ * activation pre-pass, one launch and one reduction, each with its own call's
+ * split.  Outputs equal okq_linear_out_by_in_q's on each matrix bit for bit,
+ * except those of a shared decode-batch launch, which agree within the
  * reference rule.  No counterpart in the reference,
  * whose callers compute such groups one projection at a time: the gate/up
  * pair of mlp_gated_silu (crates/kernels/src/lib.rs:150-162,
@@ -206,11 +206,15 @@ okq_status okq_gemv_multi(const float *x, int64_t rows, int64_t in_features, uin
 
 /* okq_gemv_multi for matrices of different formats: w_types[i] is matrix i's
  * GGML type (the layers of a Q4_K_M model store q/k in Q4_K and v in Q6_K).
- * Matrices of one format are grouped as okq_gemv_multi groups them; at
- * decode-batch row counts (up to 32) the Q4_K and Q6_K matrices that
- * okq_linear_out_by_in_q gives to the MFMA kernels share one decode-batch
- * launch, whose outputs agree with each matrix's own call within the
- * reference rule.  Validation and errors as okq_gemv_multi.  No counterpart in
+ * Matrices of one format are grouped as okq_gemv_multi groups them, and across
+ * formats: a single row of Q4_K and Q6_K matrices of a few rows per wave (q, k
+ * and v; not a vocabulary head) takes one GEMV launch, bit for bit each
+ * matrix's own; at decode-batch row counts (up to 32) the Q4_K and Q6_K
+ * matrices that okq_linear_out_by_in_q gives to the MFMA kernels share one
+ * decode-batch launch, whose outputs agree with each matrix's own call within
+ * the reference rule; above 32 rows the matrices of every format share one
+ * activation pre-pass and one reduction, bit for bit each matrix's own call.
+ * Validation and errors as okq_gemv_multi.  No counterpart in
  * the reference (its callers compute q, k and v one linear at a time). */
 okq_status okq_linear_multi_q(const float *x, int64_t rows, int64_t in_features, int count, const uint32_t *w_types,
                               const void *const *w, const uint64_t *w_bytes, const int64_t *out_features,
@@ -232,9 +236,11 @@ okq_status okq_rmsnorm(const float *x, int64_t rows, int64_t hidden, const float
  *   out[i][r, o] = bias[i][o] + sum_k rmsnorm(x)[r, k] * W_i[o, k].
  * Arguments as okq_rmsnorm and okq_gemv_multi.  A single row runs the GEMV
  * with the normalisation folded into its activation prologue (no normalised
- * copy of x is written); more rows normalise into a per-stream workspace
- * first and then stream each weight once per four rows.  No counterpart in the reference, whose blocks
- * call rmsnorm and then each linear (crates/models/src/qwen/qwen2_5/prefill.rs). */
+ * copy of x is written).  Up to 32 rows are normalised into a per-stream
+ * workspace first and take okq_gemv_multi's dispatch from there; above 32 rows
+ * (hidden up to 16384) the MFMA GEMM's activation pre-pass normalises them as it
+ * reads them, once for all matrices.  No counterpart in the reference, whose
+ * blocks call rmsnorm and then each linear (crates/models/src/qwen/qwen2_5/prefill.rs). */
 okq_status okq_rmsnorm_linear_q_multi(const float *x, int64_t rows, int64_t hidden, const float *norm_weight,
                                       float epsilon, uint32_t w_type, int count, const void *const *w,
                                       const uint64_t *w_bytes, const int64_t *out_features, const float *const *bias,

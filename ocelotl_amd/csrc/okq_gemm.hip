@@ -1332,10 +1332,12 @@ __global__ __launch_bounds__(kDecWaves * 64) void gemm_decode_kernel(const void 
 // rscale == nullptr) and the bias: Y[m, n] = (sum_z P[z][m, n]) * rscale[m] + bias[n].
 // Grid: 256-column blocks x rows (a row stride of gridDim.y beyond 65535
 // rows), so no thread divides its index.  The partials are read through a
-// range-checked buffer resource with 32-bit offsets (K is split only for
-// output grids under 3/4 of the CUs' tiles: at most 8 slices of a few
-// million floats), KB slices per batch, the split rounded up to 2, 4 or 8,
-// slices past it pointed at the end, where they read zeros without a branch.
+// range-checked buffer resource with 32-bit offsets (the launchers refuse
+// partials of 4 GiB; gemm_plan keeps f32 activations' below kMostPartBytes or
+// the static scratch, and splits others only on grids that leave CUs idle, at
+// most 8 ways), KB slices per batch (a split of up to 8 in one batch of 2,
+// 4 or 8, more in batches of 8), slices past it pointed at the end, where they
+// read zeros without a branch.
 template <int KB>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restrict__ part, int ksplit, int M, int N,
                                                             const float *__restrict__ rscale,
@@ -1611,10 +1613,12 @@ constexpr int64_t kMostSlices = 16;
 constexpr size_t kMostPartBytes = 192u << 20;
 
 // K slices of gemm_f32_kernel for one matrix: the split of least estimated
-// time.  A round of workgroups (one per CU) takes ~7 us (Q4_K, both planes;
-// one plane: the MFMAs of one) per super-block of its slice and ~5 us around
-// its loop; the partials are written and read once at ~4 TB/s, and their
-// reduction is one more launch.
+// time.  A round of workgroups (one per CU) takes ~7 us (Q4_K and Q5_K, both
+// planes; Q8_0 8.5, with a fold per block; Q6_K 10, with a third MFMA) per
+// super-block of its slice on 128-row tiles, 0.2 of it for what does not scale
+// with the tile's height and 0.2 per 32-row block, with one plane 0.7 of that,
+// and ~5 us around its loop; the partials are written and read once at ~4 TB/s,
+// and their reduction is one more launch.
 static int64_t f32_split(int type, int64_t M, int64_t N, int64_t K, bool one_plane, size_t part_limit, int cu_count) {
   const double us_sb = (type == kQ6_K ? 10.0 : type == kQ8_0 ? 8.5 : 7.0) * (one_plane ? 0.7 : 1.0) *
                        (0.2 + 0.2 * gemm_f32_blocks(M));
@@ -2060,7 +2064,6 @@ hipError_t launch_prefill_multi(const void *x, int64_t M, int64_t K, int count, 
 hipError_t launch_gemm(int type, const void *x, bool x_is_bf16, int64_t M, int64_t K, const void *w, int64_t N,
                        const float *bias, float *y, void *workspace, const GemmPlan &plan, hipStream_t s) {
   if (type != kQ4_K && type != kQ5_K && type != kQ6_K && type != kQ8_0) return hipErrorInvalidValue;
-  if (type != kQ4_K && type != kQ5_K && plan.bm != 128 && plan.bm != kDecRows) return hipErrorInvalidValue;
   char *ws = static_cast<char *>(workspace);
   const uint8_t *W = static_cast<const uint8_t *>(w);
   const int m = (int)M, n = (int)N, ks = plan.ksplit;

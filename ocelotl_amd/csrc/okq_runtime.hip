@@ -655,8 +655,9 @@ static okq_status prefill_multi(const float *x, int64_t rows, int64_t K, int cou
 // or more MFMA matrices at a decode-batch size share one decode-batch launch
 // (gate/up: one activation staging, one reduction); its K split follows the
 // combined columns, so those outputs match each matrix's own call within
-// the reference rule rather than bit for bit.  A single MFMA matrix, or
-// larger batches, run through okq_linear_out_by_in_q's own dispatch.
+// the reference rule rather than bit for bit.  Two or more at larger batches
+// share prefill_multi; a single MFMA matrix runs through
+// okq_linear_out_by_in_q's own dispatch.
 // swiglu_pair (count 2: gate then up of a gated-SiLU MLP): when both take one
 // decode-batch launch, its K split's reduction, or the launch itself where its
 // tiles go in pairs (gemm_decode_pairs), also applies the SiLU (out[0] =
@@ -756,11 +757,12 @@ okq_status okq_gemv_multi(const float *x, int64_t rows, int64_t in_features, uin
 }
 
 // Projections of mixed formats that read the same activations (q/k in Q4_K
-// and v in Q6_K in a Q4_K_M layer).  The Q4_K and Q6_K matrices that the
-// linear dispatch gives to the MFMA kernels share one decode-batch launch at
-// up to 32 rows (workgroups of either format, one activation staging per
-// workgroup, one reduction); everything else runs through okq_gemv_multi's
-// grouping, one format at a time.
+// and v in Q6_K in a Q4_K_M layer).  One row: the Q4_K and Q6_K matrices share
+// one GEMV launch where gemv_mixes.  Up to 32 rows: those that the linear
+// dispatch gives to the MFMA kernels share one decode-batch launch (workgroups
+// of either format, one activation staging per workgroup, one reduction).
+// Above 32 rows: the MFMA matrices of every format share prefill_multi.
+// Everything else runs through okq_gemv_multi's grouping, one format at a time.
 okq_status okq_linear_multi_q(const float *x, int64_t rows, int64_t in_features, int count, const uint32_t *w_types,
                               const void *const *w, const uint64_t *w_bytes, const int64_t *out_features,
                               const float *const *bias, float *const *out, void *stream) {

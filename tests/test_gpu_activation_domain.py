@@ -116,7 +116,7 @@ def test_gemv_intra_run_outliers_within_reference_rule(torch, okq, orc, weights,
 @pytest.mark.parametrize("rows", [2, 3, 8, 32, 64])
 def test_linear_intra_run_outliers_every_row_count(torch, okq, orc, weights, t, rows):
     """okq_linear_out_by_in_q at every row-count class (the multi-row GEMV,
-    the decode-batch MFMA kernel, the tiled GEMM) with x1000 outlier channels
+    the decode-batch MFMA kernel, the prefill GEMM) with x1000 outlier channels
     in every row."""
     n, k = 4096, 4096
     wq = weights[(t, n, k)]
@@ -224,8 +224,8 @@ NONFINITE_BATCH = [
     # prefill (
     # the register-dequant kernels (bf16 Q4_K, whole tiles and split K
     # through the reduction; bf16 Q8_0, whose bf16 MFMAs and f32 fold carry
-    # the infinities themselves, split and unsplit), the tiled kernel (f32,
-    # other formats), the pre-pass's two-pass form (K > 16384)
+    # the infinities themselves, split and unsplit), the f32 prefill kernel,
+    # the pre-pass's two-pass form (K > 16384)
     ("okq_gemm_bf16", O.Q4_K, 512, 14336, 4096),
     ("okq_gemm_bf16", O.Q4_K, 512, 4096, 14336),
     ("okq_gemm_bf16", O.Q4_K, 130, 14336, 4096),

@@ -112,7 +112,7 @@ def test_gemm_one_hot_columns_are_exact(torch, okq, orc):
 
 def test_gemm_is_deterministic_and_row_independent(torch, okq, orc):
     """Same inputs, same bits; and a row's result does not depend on the
-    other rows of its batch within a kernel family: the tiled kernel (more
+    other rows of its batch within a kernel family: a prefill kernel (more
     than 32 rows) and the decode-batch kernel (up to 32 rows) each sum a
     row's products in one fixed order (the two families' orders differ, so
     across the boundary results agree within the rule only)."""
@@ -122,7 +122,7 @@ def test_gemm_is_deterministic_and_row_independent(torch, okq, orc):
     a = run(torch, okq, "okq_gemm_bf16", O.Q4_K, xb, rows, k, wq, n)
     b = run(torch, okq, "okq_gemm_bf16", O.Q4_K, xb, rows, k, wq, n)
     assert (a.view(np.uint32) == b.view(np.uint32)).all()
-    # tiled: rows 100..163 on their own equal the same rows of the big batch
+    # prefill: rows 100..163 on their own equal the same rows of the big batch
     sub = run(torch, okq, "okq_gemm_bf16", O.Q4_K, xb.reshape(rows, k)[100:164].reshape(-1), 64, k, wq, n)
     assert (sub.view(np.uint32) == a[100:164].view(np.uint32)).all()
     # decode-batch kernel: a row alone equals the same row among 12
@@ -467,19 +467,21 @@ def test_linear_dispatch_takes_the_q6k_gemm_above_eight_rows(torch, okq, orc):
 
 
 # ---- Q8_0 -----------------------------------------------------------------------
-# f32 activations (tiled kernel): B = d * q (d the block's fp16 scale, q its
-# int8 quant) enters as two exact fp16 planes, fp16(d * q) and the remainder
-# d * q - fp16(d * q): the products are exact as for the K-quants, and no
-# per-block scaling follows.  bf16 activations above 32 rows (gemm_q8_kernel):
-# x and q enter bf16 MFMAs as they are (exact products), each block's f32 sum
-# is scaled by d; ragged tiles, split and unsplit K, K of one stage pair.
+# Decode batches: B = d * q (d the block's fp16 scale, q its int8 quant) enters
+# as two exact fp16 planes, fp16(d * q) and the remainder d * q - fp16(d * q):
+# the products are exact as for the K-quants, and no per-block scaling follows.
+# f32 activations above 32 rows (gemm_f32_kernel): q enters exactly, against the
+# activations' two fp16 planes, and each block's f32 sum is scaled by d.  bf16
+# activations above 32 rows (gemm_q8_kernel): x and q enter bf16 MFMAs as they
+# are (exact products), each block's f32 sum is scaled by d; ragged tiles, split
+# and unsplit K, K of one stage pair.
 
 Q80_CASES = [
     # decode batches (one or two 16-row MFMA groups, split and unsplit K)
     ("okq_gemm", 1, 96, 256), ("okq_gemm", 5, 300, 1024), ("okq_gemm", 8, 4096, 4096), ("okq_gemm", 16, 1000, 768),
     ("okq_gemm", 13, 4096, 14336), ("okq_gemm_bf16", 3, 14336, 4096), ("okq_gemm", 32, 4096, 4096),
     ("okq_gemm", 24, 20000, 4096), ("okq_gemm", 2, 70003, 256), ("okq_gemm_bf16", 31, 257, 768),
-    # tiled GEMM (odd block counts per tile row: 2-byte aligned block starts alternate)
+    # prefill (odd block counts per tile row: 2-byte aligned block starts alternate)
     ("okq_gemm_bf16", 33, 300, 1024), ("okq_gemm_bf16", 130, 1024, 4096), ("okq_gemm_bf16", 128, 4096, 14336),
     ("okq_gemm", 100, 257, 768), ("okq_gemm", 64, 4096, 4096), ("okq_gemm_bf16", 200, 1001, 256),
     ("okq_gemm_bf16", 200, 4096, 4096), ("okq_gemm_bf16", 130, 1000, 2048), ("okq_gemm_bf16", 64, 300, 256),
@@ -536,7 +538,7 @@ def test_gemm_q8_0_bf16_rows_of_every_m_tile(torch, okq, orc, rows, n, k):
 
 def test_gemm_q8_0_one_hot_columns_are_exact(torch, okq, orc):
     """x = e_j returns d * q of every weight row bit for bit (hi + lo = d * q
-    exactly), on the decode-batch (16 rows) and tiled (40 rows) kernels, with
+    exactly), on the decode-batch (16 rows) and prefill (40 rows) kernels, with
     scales up to d = 500 (|d * q| up to 63500) in some blocks."""
     n, k = 64, 512
     wq = orc.quantize(O.Q8_0, orc.normal(1860, n * k, 0.02))
@@ -645,8 +647,8 @@ def test_gemm_wide_one_hot_columns_are_exact(torch, okq, orc):
 # ---- Q5_K ------------------------------------------------------------------------
 # Q4_K with a fifth bit per weight (qh): B = sc * q with q <= 31, so sc * q <=
 # 1953 stays an exact fp16 integer and every product is exact as for Q4_K.
-# The decode-batch kernel (DecQ5K), the tiled kernel (f32 activations) and
-# the register-dequant kernels (bf16 activations) take it.
+# The decode-batch kernel (DecQ5K) and the register-dequant prefill kernels
+# (gemm_f32_kernel for f32 activations, the wide and pair kernels for bf16) take it.
 
 Q5K_CASES = [
     # decode batches: one and two 16-row groups, split and unsplit K, ragged N
@@ -654,7 +656,7 @@ Q5K_CASES = [
     ("okq_gemm", 13, 4096, 14336), ("okq_gemm_bf16", 3, 14336, 4096), ("okq_gemm", 6, 8000, 4096),
     ("okq_gemm", 17, 300, 1024), ("okq_gemm", 32, 4096, 4096), ("okq_gemm_bf16", 25, 1000, 768),
     ("okq_gemm", 2, 70001, 256), ("okq_gemm", 32, 300, 32768),
-    # tiled GEMM: 128-row tiles (f32 with the lo plane, bf16) and 256-row tiles (bf16 above 128 rows)
+    # prefill: f32 on 64- and 128-row tiles (every height: test_gpu_prefill_f32.py), bf16 on 128-row tiles
     ("okq_gemm", 33, 300, 1024), ("okq_gemm", 100, 257, 768), ("okq_gemm_bf16", 40, 1000, 512),
     ("okq_gemm_bf16", 130, 1024, 4096), ("okq_gemm_bf16", 300, 4096, 14336), ("okq_gemm", 64, 4096, 4096),
 ]
@@ -689,7 +691,7 @@ def test_gemm_q5k_prefill_c4_gate_sampled_rows(torch, okq, orc, rows):
 
 def test_gemm_q5k_one_hot_columns_are_exact(torch, okq, orc):
     """x = e_j picks column j of every weight row: every Q5_K path (GEMV, the
-    decode-batch kernel at 16 rows, the tiled kernel at 40 rows, f32 and
+    decode-batch kernel at 16 rows, the prefill kernels at 40 rows, f32 and
     bf16) returns the dequantized value bit for bit, with the fifth bit set
     on part of the columns."""
     n, k = 64, 512
@@ -710,8 +712,8 @@ def test_gemm_q5k_one_hot_columns_are_exact(torch, okq, orc):
 def test_gemm_q5k_fifth_bit_probe(torch, okq, orc):
     """Blocks whose only non-zero quant bit is the fifth (qs = 0, one qh bit
     set, d = 1, sc = 1, dmin = 0): the value 16 must land at exactly the
-    element the bit names, on the GEMV, the decode-batch kernel, the tiled
-    kernel (f32) and the register-dequant kernels (bf16: the 4-wave pair
+    element the bit names, on the GEMV, the decode-batch kernel and the
+    prefill kernels (f32: gemm_f32_kernel; bf16: the 4-wave pair
     kernel at 40 rows, the 8-wave wide kernel at 256), so that a misplaced
     bit plane or chunk shift moves or drops it."""
     k = 256
@@ -740,7 +742,7 @@ def test_gemm_q5k_fifth_bit_probe(torch, okq, orc):
 def test_linear_dispatch_routes_q5k_like_q4k(torch, okq, orc):
     """okq_linear_out_by_in_q on Q5_K weights: up to 8 rows the GEMV (a
     36.7 MB 4096 x 14336 weight from 3 rows the decode-batch kernel), 9-32
-    rows the decode-batch kernel, above 32 the tiled kernel; each bit for bit
+    rows the decode-batch kernel, above 32 the prefill kernel; each bit for bit
     equal to the pinned entry point and within the rule of the reference."""
     _dispatch_pairs(torch, okq, orc, O.Q5_K, 256, 1024, 2170,
                     ((8, "okq_gemv"), (9, "okq_gemm"), (40, "okq_gemm")))

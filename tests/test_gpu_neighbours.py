@@ -13,6 +13,7 @@ import ctypes
 import numpy as np
 import pytest
 
+import plan_query
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -39,6 +40,10 @@ def okq(torch):
 @pytest.fixture(scope="module")
 def orc():
     return O.Oracle()
+
+
+def _cus(torch):
+    return torch.cuda.get_device_properties(0).multi_processor_count
 
 
 def _stream(torch):
@@ -346,15 +351,15 @@ def test_mlp_gated_silu_q_split_reduction_applies_silu(torch, okq, orc, tgu, td,
 
 @pytest.mark.parametrize("tgu,td,rows,hidden,inter", [
     # gate and up in one decode-batch launch with unsplit K: 8, 4 and 2 tile
-    # slots per workgroup, uneven pairs per workgroup, a cut last tile
+    # slots per workgroup
     (O.Q4_K, O.Q6_K, 8, 4096, 14336), (O.Q4_K, O.Q4_K, 12, 1024, 8448), (O.Q5_K, O.Q4_K, 16, 1024, 7936),
-    (O.Q6_K, O.Q4_K, 9, 1280, 2816), (O.Q8_0, O.Q8_0, 10, 2048, 2600), (O.Q4_K, O.Q8_0, 13, 1024, 4096),
+    (O.Q6_K, O.Q4_K, 9, 1280, 2816), (O.Q8_0, O.Q8_0, 10, 2048, 2592), (O.Q4_K, O.Q8_0, 13, 1024, 4096),
 ])
 def test_mlp_gated_silu_q_paired_tiles_apply_silu(torch, okq, orc, tgu, td, rows, hidden, inter):
     """As above where gate+up keep K inside the workgroup: the launch itself
     leaves silu(gate(x)) * up(x) in gate_buf, and up(x) in up_buf bit for bit;
     a row with an infinity holds the SiLU of its IEEE outputs."""
-    inter = inter // 32 * 32
+    assert plan_query.decode_pairs(tgu, rows, inter, hidden, _cus(torch))
     print(f"[gpu] mlp paired tiles types={tgu},{td} rows={rows} hidden={hidden} inter={inter}", flush=True)
     x = orc.normal(7600 + rows, rows * hidden, 1.0).reshape(rows, hidden)
     x[3, 5] = np.inf
@@ -419,6 +424,7 @@ def test_mlp_one_row_in_pairs_matches_the_grouped_calls(torch, okq, orc, tgu, td
     caller's buffers carries anything between the launches: a capture on a
     stream that holds no workspace asks for none (no error is left behind) and
     replays to the same bits."""
+    assert plan_query.gemv_pairs(tgu, inter, hidden, _cus(torch))
     print(f"[gpu] mlp pairs types={tgu},{td} hidden={hidden} inter={inter} {special}", flush=True)
     x = orc.normal(7600 + hidden, hidden, 1.0)
     if special == "outlier":

@@ -415,7 +415,7 @@ MULTI_BATCH_CASES = [
     (O.Q6_K, 24, 1024, [33, 300], True),             # above 8 rows: every Q6_K matrix on the MFMA path
     (O.Q4_K, 32, 1024, [17, 1000, 256, 40], True),   # four matrices, ragged tiles, two 16-row groups
     (O.Q8_0, 12, 1024, [100, 64], True),             # Q8_0 above 8 rows: the MFMA kernels too
-    (O.Q4_K, 40, 1024, [300, 200], False),           # above 32 rows: each on the tiled GEMM
+    (O.Q4_K, 40, 1024, [300, 200], False),           # above 32 rows: one prefill launch, each with its own split
     (O.Q5_K, 8, 4096, [14336, 14336], True),         # a Q5_K gate/up pair at 8 rows
     (O.Q5_K, 24, 1024, [33, 300, 17], True),         # Q5_K above 8 rows: one decode-batch launch
 ]

@@ -52,6 +52,7 @@ def _linear(torch, okq, t, xd, rows, k, wd, n, bd=None, entry="okq_linear_out_by
     (33, 256, 40),      # one super-block, the 64-row tile mostly padding
     (64, 768, 255),     # a full 64-row tile, an odd number of super-blocks
     (65, 2304, 257),    # 96-row tiles, two column tiles, split K
+    (96, 512, 260),     # a full 96-row tile
     (97, 512, 512), (128, 4096, 300), (129, 1280, 96), (333, 1024, 520),
     (300, 8192, 4096),  # unsplit or long slices: Q8_0's sums wait in the output or the partials
     (1100, 7424, 4100),

@@ -49,7 +49,7 @@ PAIRS = [
     [(O.Q4_K, 32, 4096, 14336), (O.Q4_K, 24, 1024, 4096)],
     [(O.Q6_K, 32, 4096, 14336), (O.Q6_K, 16, 4096, 4096)],
     [(O.Q8_0, 32, 4096, 4096), (O.Q8_0, 20, 14336, 4096)],
-    # tiled GEMM: activation planes, sums, row scales and partials in the scratch
+    # prefill GEMM: activation planes, sums, row scales and partials in the scratch
     [(O.Q4_K, 64, 4096, 4096), (O.Q4_K, 40, 300, 1024)],
     [(O.Q6_K, 130, 1024, 4096), (O.Q6_K, 33, 96, 256)],
     # the GEMV needs no scratch
@@ -149,7 +149,7 @@ def test_noalloc_under_graph_capture_on_a_fresh_stream(torch, okq, orc):
 
 
 def test_noalloc_refuses_scratch_beyond_the_static_array(torch, okq, orc):
-    """4096 f32 rows of 4096: the tiled GEMM's two fp16 planes alone are
+    """4096 f32 rows of 4096: the prefill GEMM's two fp16 planes alone are
     64 MiB, so with the sums and partials more than the array holds:
     OKQ_E_SHAPE, output untouched."""
     t, rows, n, k = O.Q4_K, 4096, 256, 4096
